@@ -27,8 +27,7 @@ static_assert(kTileThreads % 64 == 0 && kTileThreads <= 1024, "a tile is whole w
 
 struct LsWork {
     double *va, *vb;      // fixed-point buffers (ghosted grid)
-    double *ex, *ey;      // extension buffers (ghosted grid), ping
-    double *fx, *fy;      // extension buffers, pong
+    double *ex, *ey;      // extension values, open marks until they are final (ghosted grid)
     int *iface, *cand, *pband;  // point lists
     unsigned char *mark;  // dilation scratch
     unsigned char *cflag; // 1 where a point takes part in the march
@@ -37,7 +36,7 @@ struct LsWork {
     int ntx, nty;         // tile grid
     int *cnt;             // counters (kCntIter + kIterSlots ints)
     int *hcnt;            // pinned host mirror
-    int pred_fim = 2, pred_ext = 2;  // passes the last march / extension needed
+    int pred_fim = 2, pred_ext = 1;  // passes the last march / extension needed
     // window of the next rebuild (see rebuild_common): level-set points
     // [win0,win1) x [win2,win3); bbox of the last band on the device, its
     // host copy and the event that marks the copy done
@@ -63,13 +62,13 @@ struct LsBatch {
     void *d_items = nullptr, *h_items = nullptr;
     int *d_cnt = nullptr, *h_cnt = nullptr;
     int cap = 0;
-    // per-solid items of the shared set-up, finish and copy launches: four
-    // regions (set-up, finish, copy-in, copy-out) in pinned memory and on
-    // the device, each rewritten only after its last upload has run
+    // per-solid items of the shared set-up and finish launches: two
+    // regions in pinned memory and on the device, each rewritten only after
+    // its last upload has run
     void *d_setup = nullptr, *h_setup = nullptr;
     size_t setup_stride = 0;
-    hipEvent_t ev_setup[4] = {nullptr, nullptr, nullptr, nullptr};
-    bool setup_used[4] = {false, false, false, false};
+    hipEvent_t ev_setup[2] = {nullptr, nullptr};
+    bool setup_used[2] = {false, false};
 };
 int ls_batch_alloc(int cap, LsBatch &bt);
 void ls_batch_free(LsBatch &bt);
