@@ -310,6 +310,15 @@ class Multigrid {
     bool dr_ = false;
     std::vector<MgLevel> L;
     size_t tail_ = 0;  // first level handled by the single-workgroup tail cycle
+    // the tail levels' coefficients (fw, fs or kc) in the tail kernel's
+    // layout, FP64 and FP32, and the coarsest level's factors (null: too
+    // large a level, swept instead)
+    double *tail_c_[2] = {nullptr, nullptr}, *tail_lu_ = nullptr;
+    float *tail_cf_[2] = {nullptr, nullptr}, *tail_luf_ = nullptr;
+    int alloc_coefs();
+    int tail_coefs(bool f32, bool copy);
+    template <class T>
+    int tail_cycle(size_t l);
     std::vector<void *> allocs;
     hipStream_t s_ = nullptr;
     double dx_ = 1, dy_ = 1;

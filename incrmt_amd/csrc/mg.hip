@@ -742,25 +742,43 @@ __global__ void k_coarse_solve(int kind, LevelArgs a, FemC k, T *z, T *b, const 
 // LDS together) runs in ONE workgroup: the levels' iterates, right-hand
 // sides, residuals and coefficients live in LDS and each smoothing colour,
 // transfer and coarse sweep is a barrier, not a kernel launch. The levels of
-// at most kTailWavePts points (the bottom of the cycle) run in the first
+// at most kTailWaveGroups groups (the bottom of the cycle) run in the first
 // wavefront alone, whose lanes synchronise without a workgroup barrier, and
-// a coarsest level of at most kTailDirect points is solved exactly by dense
-// elimination instead of by sweeps.
+// a coarsest level of at most kTailDirect points is solved exactly from the
+// factors that k_tail_coefs left.
+//
+// What bounds it is the chain of dependent phases (about 55 for MAC, 95 for
+// FEM at 32^2 and 33^2 points), so it is built for the time of one phase: a
+// thread owns a group of points on every level (a horizontal MAC pair, a 2x2
+// FEM block), reads the group's coefficients, right-hand sides and the
+// reciprocals of its diagonals into registers once per visit of a level, and
+// a phase is then the LDS reads of the neighbours' values, issued together,
+// some twenty dependent operations and one write. The coefficients of all
+// levels lie in global memory as they lie in LDS, so their load is one copy.
+// With a division in every phase, the coefficients re-read in each, run-time
+// branches on the kind and the coarsest level eliminated in every cycle, a
+// cycle of 32^2 and 33^2 points took 33.3 us on average in double precision;
+// now 14.6 (MAC) and 23.9 us (FEM), in single precision 32.2 -> 15.9 and 25.9,
+// periodic 40.1 -> 22.1 and 33.0. A phase of one
+// wavefront is about 340 (MAC) to 400 cycles (FEM), a visit's start and
+// transfer about 1200.
 constexpr int kTailMaxLev = 12;
-constexpr int kTailThreads = 1024;
+constexpr int kTailThreads = 512;   // most threads: a level's groups are at most two a thread
 constexpr int kTailArrays = 4;    // z, b, coef1, and coef2 (MAC) or r (FEM)
-constexpr int kTailWavePts = 128;
+constexpr int kTailWaveGroups = 128;
 constexpr int kTailDirect = 16;
+// the factors of the coarsest level: rows of kTailDirect, then the pivots'
+// reciprocals, then 1 where the factorisation holds
+constexpr int kTailLu = kTailDirect * kTailDirect + kTailDirect + 1;
 
 struct TailLev {
     int nx, ny, zp, off;   // LDS pitch (nx+2) and offset of the padded array
-    int gcp;               // global pitch
-    unsigned mag;          // ceil(2^20 / ((nx+1)/2)): k -> k / ((nx+1)/2) as (k * mag) >> 20
-    const void *c1, *c2;   // global coefficient arrays at (0,0): fw,fs (MAC) or kc (FEM)
+    int ha, ng;            // groups per row, groups
+    unsigned mag;          // ceil(2^20 / ha): k -> k / ha as (k * mag) >> 20
     double kx, ky;
 };
 struct TailArgs {
-    int kind, nlev, nu1, nu2, total;
+    int nlev, nu1, nu2, total;
     int wave_from;         // first level run by the first wavefront alone (nlev: none)
     int px, py;            // periodic directions (the LDS iterates keep mirrored rings)
     int dr;                // zero-pressure right edge (MAC prolongation mirrors with a sign)
@@ -769,6 +787,8 @@ struct TailArgs {
     TailLev lv[kTailMaxLev];
     void *z_top;
     const void *b_top;
+    const void *c1, *c2;   // the levels' coefficients, laid out as in LDS: fw, fs (MAC) or kc (FEM)
+    const void *lu;        // the coarsest level's factors
     int top_pitch;
     double reduce;
     int max_sweeps;
@@ -778,6 +798,22 @@ template <class T>
 __device__ inline double tail_wave_sum(double v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
+}
+// tail_wave_sum of a value that only the first 16 lanes hold (the others
+// zero): the same additions, the zeros left out, and the sum broadcast. On
+// data of period 2n within 16 lanes, rotating by n is the exchange with n.
+__device__ inline double tail_sum16(double v) {
+    auto rot = [](double x, auto c) {
+        const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+        const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)b, decltype(c)::value, 0xf, 0xf, false);
+        const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), decltype(c)::value, 0xf, 0xf, false);
+        return __longlong_as_double((long long)((unsigned long long)(unsigned)hi << 32 | (unsigned)lo));
+    };
+    v += rot(v, std::integral_constant<int, 0x128>());  // row_ror 8
+    v += rot(v, std::integral_constant<int, 0x124>());
+    v += rot(v, std::integral_constant<int, 0x122>());
+    v += rot(v, std::integral_constant<int, 0x121>());
+    return __shfl(v, 0, 64);
 }
 template <class T>
 __device__ double tail_block_sum(double v, double *red) {
@@ -791,83 +827,61 @@ __device__ double tail_block_sum(double v, double *red) {
     return s;
 }
 
-// LDS writes of a wavefront's lanes visible to its other lanes
-__device__ inline void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// LDS writes of a wavefront's lanes visible to its other lanes: the LDS runs
+// a wavefront's operations in order, so only the compiler has to keep theirs
+// (a fence would wait for every write's end, 100 cycles a phase)
+__device__ inline void wave_sync() { asm volatile("" ::: "memory"); }
+
+// n / d, correctly rounded, from y = 1 / d correctly rounded (P. Markstein,
+// IBM J. Res. Dev. 34, 1990: with q within a rounding of n / d, the remainder
+// n - d q is exact in one fused operation and q + y (n - d q) rounds to the
+// quotient; the first correction brings q there). Five dependent operations
+// instead of a division's thirty.
+__host__ __device__ inline double quot(double n, double d, double y) {
+    double q = n * y;
+    q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
+    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+__host__ __device__ inline float quot(float n, float d, float y) {
+    float q = n * y;
+    q = __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+}
+__device__ inline double read_lane(double v, int l) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, l), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), l);
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+__device__ inline float read_lane(float v, int l) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), l));
 }
 
-template <class T, bool PER>
+// A MAC pair's coefficients: the points of colour 0 and 1
+template <class T>
+struct TailMac {
+    T wl[2], wr[2], sd[2], su[2], d[2], y[2], b[2];
+    int q[2], i[2], j;
+    bool on[2], upd[2];  // on the level; updated by the sweeps (a diagonal that is not zero)
+};
+// A FEM block's: its points in colour order, the nine cells around them
+template <class T>
+struct TailFem {
+    T kc[9], d[4], y[4], b[4], z[4];
+    int q, i, j;
+    bool on[4], upd[4];
+};
+
+template <class T, int KIND, bool PER>
 __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
     const int px = PER ? A.px : 0, py = PER ? A.py : 0;
     extern __shared__ __align__(16) unsigned char smem[];
     T *pool = (T *)smem;
     __shared__ double red[16];
-    __shared__ T dm[kTailDirect * kTailDirect];  // reduced system of the direct coarsest solve
+    __shared__ T lu[kTailLu];
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63;
-    auto arr = [&](int a, int l) -> T * { return pool + a * A.total + A.lv[l].off + A.lv[l].zp + 1; };
-    // a level's LDS arrays as a LevelArgs, for put_z (mirrored periodic rings)
-    auto lds = [&](int l) -> LevelArgs {
-        const TailLev &v = A.lv[l];
-        return LevelArgs{v.nx, v.ny, v.zp, v.zp, v.kx, v.ky, px, py};
-    };
-    // an iterate write, with the periodic mirrors when the levels have them
-    auto tput = [&](const LevelArgs &la, T *arr_, int i, int j, T v) {
-        if (PER) put_z(la, arr_, i, j, v);
-        else arr_[j * la.zp + i] = v;
-    };
-    for (int p = tid; p < kTailArrays * A.total; p += nt) pool[p] = 0;
-    __syncthreads();
-    // coefficients with their zero ring (all levels as one flat range, two
-    // points per thread in flight), and the top level's z and b
-    for (int base = 0; base < A.total; base += 2 * nt) {
-        T v1[2], v2[2];
-        int dst[2];
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int p = base + u * nt + tid;
-            dst[u] = -1;
-            v1[u] = v2[u] = 0;
-            if (p < A.total) {
-                int l = 0;
-                while (l + 1 < A.nlev && p >= A.lv[l + 1].off) l++;
-                const TailLev &v = A.lv[l];
-                const int q = p - v.off, W = v.nx + 2, jj = q / W, ii = q - jj * W;
-                const int g = (jj - 1) * v.gcp + (ii - 1);
-                v1[u] = ((const T *)v.c1)[g];
-                if (A.kind == kMAC) v2[u] = ((const T *)v.c2)[g];
-                dst[u] = p;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-            if (dst[u] >= 0) {
-                pool[2 * A.total + dst[u]] = v1[u];
-                if (A.kind == kMAC) pool[3 * A.total + dst[u]] = v2[u];
-            }
-    }
-    {
-        const TailLev &v = A.lv[0];
-        const T *gb = (const T *)A.b_top, *gz = (const T *)A.z_top;
-        for (int p = tid; p < v.nx * v.ny; p += nt) {
-            const int i = p % v.nx, j = p / v.nx;
-            const T bb = gb[j * A.top_pitch + i], zz = gz[j * A.top_pitch + i];
-            arr(1, 0)[j * v.zp + i] = bb;
-            tput(lds(0), arr(0, 0), i, j, zz);
-        }
-    }
-    __syncthreads();
-    // w: the first wavefront alone (lanes 0..63, wave_sync) instead of the
-    // whole workgroup (__syncthreads)
-    auto sync = [&](bool w) {
-        if (w) wave_sync();
-        else __syncthreads();
-    };
+    const FemC kk = A.k;
     // A level's parameters and LDS arrays, read from the kernel arguments
-    // once per phase: a level index known only at run time keeps the
-    // compiler from hoisting those reads out of the conditional point
-    // updates, where each would wait on a scalar load.
+    // once per visit
     struct Lv {
         TailLev v;
         T *z, *b, *c1, *c2;
@@ -876,226 +890,365 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
     auto lvl = [&](int l) -> Lv {
         Lv L;
         L.v = A.lv[l];
-        L.z = arr(0, l); L.b = arr(1, l); L.c1 = arr(2, l); L.c2 = arr(3, l);
+        T *p = pool + L.v.off + L.v.zp + 1;
+        L.z = p; L.b = p + A.total; L.c1 = p + 2 * A.total; L.c2 = p + 3 * A.total;
         L.la = LevelArgs{L.v.nx, L.v.ny, L.v.zp, L.v.zp, L.v.kx, L.v.ky, px, py};
         return L;
     };
-    const int kind = A.kind;
-    const FemC kk = A.k;
-    auto offd = [&](const Lv &L, int i, int j, T &diag) -> T {
-        const int q = j * L.v.zp + i;
-        if (kind == kMAC) return mac_offdiag<T>(L.z, L.c1, L.c2, q, q, L.v.zp, L.v.zp, T(L.v.kx), T(L.v.ky), diag);
-        return fem_offdiag<T>(L.z, L.c1, q, q, L.v.zp, L.v.zp, kk, diag);
+    // an iterate write, with the periodic mirrors when the levels have them
+    auto tput = [&](const Lv &L, T *arr, int i, int j, T v) {
+        if (PER) put_z(L.la, arr, i, j, v);
+        else arr[j * L.v.zp + i] = v;
     };
-    // colour phases enumerate only their own points: the k-th point of a
-    // colour is in colour row r = k / ha, column a = k - r ha
-    auto smooth = [&](int l, int sweeps, bool reverse, bool w) {
-        const Lv L = lvl(l);
+    // w: the first wavefront alone (lanes 0..63, wave_sync) instead of the
+    // whole workgroup (__syncthreads)
+    auto sync = [&](bool w) {
+        if (w) wave_sync();
+        else __syncthreads();
+    };
+    const Lv top = lvl(0);
+    {
+        // every global read issued before the barrier behind which its
+        // value is written: the top level's own points, then the
+        // coefficients four at a time
+        const T *gb = (const T *)A.b_top, *gz = (const T *)A.z_top, *g1 = (const T *)A.c1, *g2 = (const T *)A.c2,
+                *gl = (const T *)A.lu;
+        constexpr int kPts = KIND == kMAC ? 2 : 4;
+        T zz[2 * kPts], bb[2 * kPts];
+        int ii[2 * kPts], jj[2 * kPts];
+#pragma unroll
+        for (int e = 0; e < 2 * kPts; e++) {
+            const int k = tid + e / kPts * nt, c = e % kPts;
+            const int r = (int)(((unsigned)k * top.v.mag) >> 20), a = k - r * top.v.ha;
+            ii[e] = 2 * a + (c & 1);
+            jj[e] = KIND == kMAC ? r : 2 * r + (c >> 1);
+            if (k >= top.v.ng || ii[e] >= top.v.nx || jj[e] >= top.v.ny) ii[e] = -1;
+            zz[e] = bb[e] = 0;
+            if (ii[e] >= 0) {
+                zz[e] = gz[jj[e] * A.top_pitch + ii[e]];
+                bb[e] = gb[jj[e] * A.top_pitch + ii[e]];
+            }
+        }
+        for (int base = tid; base < A.total; base += 4 * nt) {
+            T v1[4], v2[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int p = base + u * nt;
+                v1[u] = v2[u] = 0;
+                if (p < A.total) {
+                    v1[u] = g1[p];
+                    if (KIND == kMAC) v2[u] = g2[p];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int p = base + u * nt;
+                if (p < A.total) {
+                    pool[p] = 0;
+                    pool[2 * A.total + p] = v1[u];
+                    pool[3 * A.total + p] = v2[u];  // FEM: the residuals' zero ring
+                }
+            }
+        }
+        if (gl)
+            for (int p = tid; p < kTailLu; p += nt) lu[p] = gl[p];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 2 * kPts; e++)
+            if (ii[e] >= 0) {
+                tput(top, top.z, ii[e], jj[e], zz[e]);
+                top.b[jj[e] * top.v.zp + ii[e]] = bb[e];
+            }
+    }
+    __syncthreads();
+    // The off-diagonal sums and diagonals keep the expressions of
+    // mac_offdiag and fem_offdiag.
+    auto load_mac = [&](const Lv &L, int k) -> TailMac<T> {
+        TailMac<T> g;
         const TailLev &v = L.v;
-        const int ncol = kind == kMAC ? 2 : 4, ha = (v.nx + 1) >> 1;
-        const int N = ha * (kind == kMAC ? v.ny : (v.ny + 1) >> 1);
-        const int t0 = w ? lane : tid, st = w ? 64 : nt;
-        for (int sw = 0; sw < sweeps; sw++)
-            for (int cc = 0; cc < ncol; cc++) {
-                const int col = reverse ? ncol - 1 - cc : cc;
-                for (int k = t0; k < N; k += st) {
-                    const int r = (int)(((unsigned)k * v.mag) >> 20), a = k - r * ha;
-                    const int j = kind == kMAC ? r : 2 * r + (col >> 1);
-                    const int i = kind == kMAC ? 2 * a + ((col + j) & 1) : 2 * a + (col & 1);
-                    if (i >= v.nx || j >= v.ny) continue;
-                    T diag;
-                    const T off = offd(L, i, j, diag);
-                    if (diag != T(0)) tput(L.la, L.z, i, j, (L.b[j * v.zp + i] - off) / diag);
+        const int r = (int)(((unsigned)k * v.mag) >> 20), a = k - r * v.ha;
+        g.j = r;
+        const T kx = T(v.kx), ky = T(v.ky);
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            g.i[c] = 2 * a + ((c + r) & 1);
+            g.on[c] = k < v.ng && g.i[c] < v.nx;
+            g.q[c] = g.on[c] ? r * v.zp + g.i[c] : 0;
+            const int q = g.q[c];
+            g.wl[c] = L.c1[q]; g.wr[c] = L.c1[q + 1]; g.sd[c] = L.c2[q]; g.su[c] = L.c2[q + v.zp];
+            g.b[c] = L.b[q];
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            g.d[c] = -(kx * (g.wl[c] + g.wr[c]) + ky * (g.sd[c] + g.su[c]));
+            g.y[c] = T(1) / g.d[c];
+            g.upd[c] = g.on[c] && g.d[c] != T(0);
+        }
+        return g;
+    };
+    auto off_mac = [&](const Lv &L, const TailMac<T> &g, int c) -> T {
+        const T *z = L.z + g.q[c];
+        const int zp = L.v.zp;
+        const T zl = z[-1], zr = z[1], zd = z[-zp], zu = z[zp];
+        return T(L.v.kx) * (g.wl[c] * zl + g.wr[c] * zr) + T(L.v.ky) * (g.sd[c] * zd + g.su[c] * zu);
+    };
+    auto load_fem = [&](const Lv &L, int k) -> TailFem<T> {
+        TailFem<T> g;
+        const TailLev &v = L.v;
+        const int r = (int)(((unsigned)k * v.mag) >> 20), a = k - r * v.ha;
+        const bool mine = k < v.ng;
+        g.i = 2 * a; g.j = 2 * r;
+        g.q = mine ? g.j * v.zp + g.i : 0;
+#pragma unroll
+        for (int c = 0; c < 9; c++) g.kc[c] = L.c1[g.q + (c / 3 - 1) * v.zp + c % 3 - 1];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const int p = g.q + (c & 1) + (c >> 1) * v.zp;
+            g.on[c] = mine && g.i + (c & 1) < v.nx && g.j + (c >> 1) < v.ny;
+            g.b[c] = L.b[p];
+            g.z[c] = L.z[p];
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const T *kc = g.kc + (c >> 1) * 3 + (c & 1);
+            g.d[c] = T(kk.fm) * (kc[0] + kc[1] + kc[3] + kc[4]);
+            g.y[c] = T(1) / g.d[c];
+            g.upd[c] = g.on[c] && g.d[c] != T(0);
+        }
+        return g;
+    };
+    auto off_fem = [&](const Lv &L, const TailFem<T> &g, int c) -> T {
+        const int cx = c & 1, cy = c >> 1, zp = L.v.zp;
+        // a neighbour of the own block comes from its register (not on a
+        // periodic level, where a block past an odd edge holds a mirror of
+        // another block's point)
+        auto nb = [&](int dx, int dy) -> T {
+            const int x = cx + dx, y = cy + dy;
+            if (!PER && x >= 0 && x < 2 && y >= 0 && y < 2) return g.z[x + 2 * y];
+            return L.z[g.q + x + y * zp];
+        };
+        const T zdl = nb(-1, -1), zdr = nb(1, -1), zul = nb(-1, 1), zur = nb(1, 1), zd = nb(0, -1), zu = nb(0, 1),
+                zl = nb(-1, 0), zr = nb(1, 0);
+        const T *kc = g.kc + cy * 3 + cx;
+        const T kdl = kc[0], kdr = kc[1], kul = kc[3], kur = kc[4];
+        return T(kk.fc) * (kdl * zdl + kdr * zdr + kul * zul + kur * zur) +
+               T(kk.hey) * ((kdl + kdr) * zd + (kul + kur) * zu) + T(kk.hex) * ((kdl + kul) * zl + (kdr + kur) * zr);
+    };
+    // One visit of a level, groups t0 + st u of the first wavefront or of the
+    // workgroup. DOWN: pre-smooth, restrict the residual to the
+    // next level's right-hand side and clear its iterate; else add the next
+    // level's correction and post-smooth; SWEEP: `sweeps` forward sweeps.
+    enum { kDown, kUp, kSweep };
+    auto visit = [&](auto groups, auto what, const Lv &L, const Lv &C, bool w, int sweeps) {
+        constexpr int G = decltype(groups)::value, WHAT = decltype(what)::value;
+        const int t0 = w ? lane : tid, st = w ? 64 : nt, zp = L.v.zp;
+        if constexpr (KIND == kMAC) {
+            TailMac<T> g[G];
+#pragma unroll
+            for (int u = 0; u < G; u++) g[u] = load_mac(L, t0 + st * u);
+            if constexpr (WHAT == kUp) {
+                const int cz = C.v.zp, cnx = C.v.nx, cny = C.v.ny;
+#pragma unroll
+                for (int u = 0; u < G; u++)
+#pragma unroll
+                    for (int c = 0; c < 2; c++)
+                        if (g[u].on[c]) {
+                            const int i = g[u].i[c], j = g[u].j, I = i >> 1, J = j >> 1;
+                            int I2 = I + ((i & 1) ? 1 : -1), J2 = J + ((j & 1) ? 1 : -1);
+                            const bool flip = A.dr && I2 >= cnx;
+                            if (I2 < 0 || I2 >= cnx) I2 = px ? wrap_idx(I2, cnx) : I;
+                            if (J2 < 0 || J2 >= cny) J2 = py ? wrap_idx(J2, cny) : J;
+                            const T *e = C.z;
+                            T e2 = e[J * cz + I2], e22 = e[J2 * cz + I2];
+                            if (flip) { e2 = -e2; e22 = -e22; }
+                            const T add = T(0.5625) * e[J * cz + I] + T(0.1875) * e2 + T(0.1875) * e[J2 * cz + I] +
+                                          T(0.0625) * e22;
+                            tput(L, L.z, i, j, L.z[g[u].q[c]] + add);
+                        }
+                sync(w);
+            }
+            for (int sw = 0; sw < sweeps; sw++)
+#pragma unroll
+                for (int cc = 0; cc < 2; cc++) {
+                    const int c = WHAT == kUp ? 1 - cc : cc;
+                    // (every group computed, masked only in the write, so that
+                    // two groups' chains overlap)
+                    T z[G];
+#pragma unroll
+                    for (int u = 0; u < G; u++) z[u] = quot(g[u].b[c] - off_mac(L, g[u], c), g[u].d[c], g[u].y[c]);
+#pragma unroll
+                    for (int u = 0; u < G; u++)
+                        if (g[u].upd[c]) tput(L, L.z, g[u].i[c], g[u].j, z[u]);
+                    sync(w);
+                }
+            if constexpr (WHAT == kDown) {
+                const T kx = T(L.v.kx), ky = T(L.v.ky);
+#pragma unroll
+                for (int u = 0; u < G; u++) {
+                    const int k = t0 + st * u;
+                    if (k < C.v.nx * C.v.ny) {  // a coarse row holds as many points as a fine row pairs
+                        const int J = (int)(((unsigned)k * L.v.mag) >> 20), I = k - J * L.v.ha;
+                        const int q0 = 2 * J * zp + 2 * I;
+                        T s = 0;
+#pragma unroll
+                        for (int c = 0; c < 4; c++) {
+                            const int q = q0 + (c & 1) + (c >> 1) * zp;
+                            T diag;
+                            const T off = mac_offdiag<T>(L.z, L.c1, L.c2, q, q, zp, zp, kx, ky, diag);
+                            s += L.b[q] - off - diag * L.z[q];
+                        }
+                        C.b[J * C.v.zp + I] = T(0.25) * s;
+                        tput(C, C.z, I, J, T(0));
+                    }
                 }
                 sync(w);
             }
-    };
-    auto residual = [&](const Lv &L, int i, int j) -> T {
-        T diag;
-        const T off = offd(L, i, j, diag);
-        return L.b[j * L.v.zp + i] - off - diag * L.z[j * L.v.zp + i];
-    };
-    // pre-smooth level l, restrict its residual to l+1's right-hand side and
-    // clear l+1's iterate
-    auto down = [&](int l, bool w) {
-        smooth(l, A.nu1, false, w);
-        const Lv F = lvl(l), C = lvl(l + 1);
-        const TailLev &f = F.v, &c = C.v;
-        const int t0 = w ? lane : tid, st = w ? 64 : nt;
-        if (kind == kMAC) {
-            for (int p = t0; p < c.nx * c.ny; p += st) {
-                const int I = p % c.nx, J = p / c.nx;
-                T s = 0;
-                for (int dj = 0; dj < 2; dj++)
-                    for (int di = 0; di < 2; di++) s += residual(F, 2 * I + di, 2 * J + dj);
-                C.b[J * c.zp + I] = T(0.25) * s;
-                tput(C.la, C.z, I, J, T(0));
-            }
         } else {
-            for (int p = t0; p < f.nx * f.ny; p += st) {
-                const int i = p % f.nx, j = p / f.nx;
-                tput(F.la, F.c2, i, j, residual(F, i, j));
+            TailFem<T> g[G];
+#pragma unroll
+            for (int u = 0; u < G; u++) g[u] = load_fem(L, t0 + st * u);
+            if constexpr (WHAT == kUp) {
+#pragma unroll
+                for (int u = 0; u < G; u++)
+                    if (g[u].on[0]) {
+                        const T *e = C.z + (g[u].j >> 1) * C.v.zp + (g[u].i >> 1);
+                        const T e0 = e[0], e1 = e[1], e2 = e[C.v.zp], e3 = e[C.v.zp + 1];
+                        const T add[4] = {e0, T(0.5) * (e0 + e1), T(0.5) * (e0 + e2), T(0.25) * (e0 + e1 + e2 + e3)};
+#pragma unroll
+                        for (int c = 0; c < 4; c++)
+                            if (g[u].on[c]) {
+                                g[u].z[c] = g[u].z[c] + add[c];
+                                tput(L, L.z, g[u].i + (c & 1), g[u].j + (c >> 1), g[u].z[c]);
+                            }
+                    }
+                sync(w);
             }
-            sync(w);
-            const T *r = F.c2;
-            const int pz = f.zp;
-            for (int p = t0; p < c.nx * c.ny; p += st) {
-                const int I = p % c.nx, J = p / c.nx, q = 2 * J * pz + 2 * I;
-                C.b[J * c.zp + I] = r[q] + T(0.5) * (r[q - 1] + r[q + 1] + r[q - pz] + r[q + pz])
-                                    + T(0.25) * (r[q - pz - 1] + r[q - pz + 1] + r[q + pz - 1] + r[q + pz + 1]);
-                tput(C.la, C.z, I, J, T(0));
+            for (int sw = 0; sw < sweeps; sw++)
+#pragma unroll
+                for (int cc = 0; cc < 4; cc++) {
+                    const int c = WHAT == kUp ? 3 - cc : cc;
+                    T z[G];
+#pragma unroll
+                    for (int u = 0; u < G; u++) z[u] = quot(g[u].b[c] - off_fem(L, g[u], c), g[u].d[c], g[u].y[c]);
+#pragma unroll
+                    for (int u = 0; u < G; u++)
+                        if (g[u].upd[c]) {
+                            g[u].z[c] = z[u];
+                            tput(L, L.z, g[u].i + (c & 1), g[u].j + (c >> 1), z[u]);
+                        }
+                    sync(w);
+                }
+            if constexpr (WHAT == kDown) {
+#pragma unroll
+                for (int u = 0; u < G; u++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+                        if (g[u].on[c])
+                            tput(L, L.c2, g[u].i + (c & 1), g[u].j + (c >> 1),
+                                 g[u].b[c] - off_fem(L, g[u], c) - g[u].d[c] * g[u].z[c]);
+                sync(w);
+                const T *r = L.c2;
+#pragma unroll
+                for (int u = 0; u < G; u++)
+                    if (g[u].on[0] && (g[u].i >> 1) < C.v.nx && (g[u].j >> 1) < C.v.ny) {
+                        // the block's first point is the coarse node
+                        const int q = g[u].q;
+                        C.b[(g[u].j >> 1) * C.v.zp + (g[u].i >> 1)] =
+                            r[q] + T(0.5) * (r[q - 1] + r[q + 1] + r[q - zp] + r[q + zp]) +
+                            T(0.25) * (r[q - zp - 1] + r[q - zp + 1] + r[q + zp - 1] + r[q + zp + 1]);
+                        tput(C, C.z, g[u].i >> 1, g[u].j >> 1, T(0));
+                    }
+                sync(w);
             }
         }
-        sync(w);
     };
-    // add level l+1's correction to level l and post-smooth level l
-    auto up = [&](int l, bool w) {
-        const Lv F = lvl(l), C = lvl(l + 1);
-        const TailLev &f = F.v, &c = C.v;
-        const T *e = C.z;
-        const int p2 = c.zp, t0 = w ? lane : tid, st = w ? 64 : nt;
-        const bool dr = A.dr;
-        for (int p = t0; p < f.nx * f.ny; p += st) {
-            const int i = p % f.nx, j = p / f.nx, I = i >> 1, J = j >> 1;
-            T add;
-            if (kind == kMAC) {
-                int I2 = I + ((i & 1) ? 1 : -1), J2 = J + ((j & 1) ? 1 : -1);
-                const bool flip = dr && I2 >= c.nx;
-                if (I2 < 0 || I2 >= c.nx) I2 = px ? wrap_idx(I2, c.nx) : I;
-                if (J2 < 0 || J2 >= c.ny) J2 = py ? wrap_idx(J2, c.ny) : J;
-                T e2 = e[J * p2 + I2], e22 = e[J2 * p2 + I2];
-                if (flip) { e2 = -e2; e22 = -e22; }
-                add = T(0.5625) * e[J * p2 + I] + T(0.1875) * e2 + T(0.1875) * e[J2 * p2 + I] + T(0.0625) * e22;
-            } else {
-                const int q = J * p2 + I;
-                if (!(i & 1) && !(j & 1)) add = e[q];
-                else if (!(j & 1)) add = T(0.5) * (e[q] + e[q + 1]);
-                else if (!(i & 1)) add = T(0.5) * (e[q] + e[q + p2]);
-                else add = T(0.25) * (e[q] + e[q + 1] + e[q + p2] + e[q + p2 + 1]);
-            }
-            tput(F.la, F.z, i, j, F.z[j * f.zp + i] + add);
-        }
-        sync(w);
-        smooth(l, A.nu2, true, w);
+    auto run = [&](auto what, const Lv &L, const Lv &C, bool w, int sweeps) {
+        if (L.v.ng > (w ? 64 : nt)) visit(std::integral_constant<int, 2>(), what, L, C, w, sweeps);
+        else visit(std::integral_constant<int, 1>(), what, L, C, w, sweeps);
     };
     // Exact solve of a coarsest level of N <= kTailDirect points by the first
-    // wavefront. A pure-Neumann level has a mean-free, hence compatible,
-    // right-hand side and a symmetric operator with the constants as its null
-    // space, so fixing point 0 at zero leaves a definite system in points
-    // 1..N-1 (o = 1); a definite level keeps all N points (o = 0). Eliminated
-    // without pivoting (row r of dm is point r+o). False (nothing written)
-    // when a pivot is zero, not finite or of the other sign.
-    auto direct = [&](int l) -> bool {
-        const Lv L = lvl(l);
-        const TailLev &v = L.v;
-        const int o = A.sing ? 1 : 0, N = v.nx * v.ny, n = N - o;
-        if (lane < n) {
-            const int p = lane + o, i = p % v.nx, j = p / v.nx, q = j * v.zp + i;
-            T *row = dm + lane * kTailDirect;
-            for (int c = 0; c < kTailDirect; c++) row[c] = 0;
-            auto put = [&](int di, int dj, T a) {
-                int ii = i + di, jj = j + dj;
-                if (px) ii = wrap_idx(ii, v.nx);
-                if (py) jj = wrap_idx(jj, v.ny);
-                if (ii < 0 || ii >= v.nx || jj < 0 || jj >= v.ny) return;
-                const int pn = jj * v.nx + ii;
-                if (pn >= o) row[pn - o] += a;
-            };
-            if (kind == kMAC) {
-                const T *fw = L.c1, *fs = L.c2, kx = T(v.kx), ky = T(v.ky);
-                const T wl = fw[q], wr = fw[q + 1], sd = fs[q], su = fs[q + v.zp];
-                put(0, 0, -(kx * (wl + wr) + ky * (sd + su)));
-                put(-1, 0, kx * wl);
-                put(1, 0, kx * wr);
-                put(0, -1, ky * sd);
-                put(0, 1, ky * su);
-            } else {
-                const T *kc = L.c1;
-                const T kdl = kc[q - v.zp - 1], kdr = kc[q - v.zp], kul = kc[q - 1], kur = kc[q];
-                put(0, 0, T(kk.fm) * (kdl + kdr + kul + kur));
-                put(-1, -1, T(kk.fc) * kdl);
-                put(1, -1, T(kk.fc) * kdr);
-                put(-1, 1, T(kk.fc) * kul);
-                put(1, 1, T(kk.fc) * kur);
-                put(0, -1, T(kk.hey) * (kdl + kdr));
-                put(0, 1, T(kk.hey) * (kul + kur));
-                put(-1, 0, T(kk.hex) * (kdl + kul));
-                put(1, 0, T(kk.hex) * (kdr + kur));
+    // wavefront, all in registers: lane p holds point p, and its row of the
+    // factors (k_tail_coefs; a pure-Neumann level has point 0 fixed at zero,
+    // o = 1, and gets a mean-free right-hand side and iterate): forward and
+    // back substitution, a step one broadcast.
+    auto direct = [&](auto size, const Lv &L) {
+        constexpr int M = decltype(size)::value;
+        const int o = A.sing ? 1 : 0, N = L.v.nx * L.v.ny, n = N - o, r = lane - o;
+        int j = 0, i = lane;  // lane = j nx + i
+        for (int k = 0; k + 1 < L.v.ny; k++)
+            if (i >= L.v.nx) {
+                i -= L.v.nx;
+                j++;
             }
+        const bool mine = lane < N, solved = mine && r >= 0;
+        T row[M], rhs = 0, piv = 1, y = 1, x = 0, xs[M];
+        if (mine) rhs = L.b[j * L.v.zp + i];
+#pragma unroll
+        for (int c = 0; c < M; c++) {
+            row[c] = solved && c < n ? lu[r * kTailDirect + c] : T(0);
+            xs[c] = 0;
         }
-        // lane r keeps row r's right-hand side in a register
-        T rhs = 0;
-        if (lane < n) {
-            const int p = lane + o;
-            rhs = L.b[(p / v.nx) * v.zp + p % v.nx];
+        if (solved) {
+            piv = lu[r * kTailDirect + r];
+            y = lu[kTailDirect * kTailDirect + r];
         }
-        wave_sync();
-        bool ok = true;
-        T s0 = 0;
-        for (int k = 0; k < n; k++) {
-            const T piv = dm[k * kTailDirect + k];
-            if (k == 0) s0 = piv;
-            if (!(piv == piv) || piv == T(0) || (piv > T(0)) != (s0 > T(0)) || !(piv * T(0) == T(0))) {
-                ok = false;
-                break;
-            }
-            const T rk = __shfl(rhs, k, 64);
-            if (lane > k && lane < n) {
-                const T f = dm[lane * kTailDirect + k] / piv;
-                for (int c = k + 1; c < n; c++) dm[lane * kTailDirect + c] -= f * dm[k * kTailDirect + c];
-                rhs -= f * rk;
-            }
-            wave_sync();
+        if (A.sing) rhs -= T(tail_sum16(double(rhs)) / N);
+#pragma unroll
+        for (int k = 0; k < M; k++) {
+            const T rk = read_lane(rhs, k + o);
+            if (r > k && solved) rhs -= row[k] * rk;
         }
-        if (!ok) return false;
-        // back substitution, one unknown at a time from the last
-        T x = 0;
-        for (int k = n - 1; k >= 0; k--) {
-            // lane k owns row k; the unknowns after it are already in x of their lanes
+#pragma unroll
+        for (int k = M - 1; k >= 0; k--) {
+            // (past the last unknown every factor and value is zero)
             T acc = 0;
-            for (int c = k + 1; c < n; c++) acc += dm[k * kTailDirect + c] * __shfl(x, c, 64);
-            const T xk = (__shfl(rhs, k, 64) - acc) / dm[k * kTailDirect + k];
-            if (lane == k) x = xk;
+#pragma unroll
+            for (int c = k + 1; c < M; c++) acc += row[c] * xs[c];
+            const T xk = quot(rhs - acc, piv, y);
+            if (r == k && solved) x = xk;
+            xs[k] = k < n ? read_lane(xk, k + o) : T(0);
         }
-        if (lane < n) {
-            const int p = lane + o;
-            tput(L.la, L.z, p % v.nx, p / v.nx, x);
-        }
-        // the pinned point 0 (a warm-started single-level tail holds an
-        // iterate there)
-        if (o && lane == 0) tput(L.la, L.z, 0, 0, T(0));
+        if (A.sing) x -= T(tail_sum16(mine ? double(x) : 0.0) / N);
+        if (mine) tput(L, L.z, i, j, x);
         wave_sync();
-        return true;
     };
     // coarsest: mean-free right-hand side, then the direct solve or sweeps to
     // a residual reduction, then a mean-free iterate (pure Neumann; a
     // definite level skips both projections)
-    auto coarsest = [&](bool w) {
-        const int l = A.nlev - 1;
-        const Lv L = lvl(l);
+    auto coarsest = [&](const Lv &L, bool w) {
         const TailLev &v = L.v;
-        const int N = v.nx * v.ny, t0 = w ? lane : tid, st = w ? 64 : nt;
+        const int N = v.nx * v.ny, n = N - (A.sing ? 1 : 0), t0 = w ? lane : tid, st = w ? 64 : nt;
+        if (w && A.lu && lu[kTailLu - 1] != T(0)) {
+            if (n <= 4) direct(std::integral_constant<int, 4>(), L);
+            else if (n <= 8) direct(std::integral_constant<int, 8>(), L);
+            else direct(std::integral_constant<int, 16>(), L);
+            return;
+        }
         auto total = [&](double a) -> double { return w ? tail_wave_sum<T>(a) : tail_block_sum<T>(a, red); };
         double sb = 0;
         for (int p = t0; p < N; p += st) sb += double(L.b[(p / v.nx) * v.zp + p % v.nx]);
         const T mb = A.sing ? T(total(sb) / N) : T(0);
         for (int p = t0; p < N; p += st) L.b[(p / v.nx) * v.zp + p % v.nx] -= mb;
         sync(w);
-        const bool solved = w && N <= kTailDirect && N > 1 && direct(l);
-        if (!solved) {
-            auto r2 = [&]() -> double {
-                double a = 0;
-                for (int p = t0; p < N; p += st) {
-                    const double r = double(residual(L, p % v.nx, p / v.nx));
-                    a += r * r;
-                }
-                return total(a);
-            };
-            const double r0 = r2();
-            for (int it = 0; it < A.max_sweeps && r0 > 0; it++) {
-                smooth(l, 1, false, w);
-                if ((it & 7) == 7 && r2() <= A.reduce * A.reduce * r0) break;
+        auto residual = [&](int i, int j) -> T {
+            const int q = j * v.zp + i;
+            T diag;
+            const T off = KIND == kMAC ? mac_offdiag<T>(L.z, L.c1, L.c2, q, q, v.zp, v.zp, T(v.kx), T(v.ky), diag)
+                                       : fem_offdiag<T>(L.z, L.c1, q, q, v.zp, v.zp, kk, diag);
+            return L.b[q] - off - diag * L.z[q];
+        };
+        auto r2 = [&]() -> double {
+            double a = 0;
+            for (int p = t0; p < N; p += st) {
+                const double r = double(residual(p % v.nx, p / v.nx));
+                a += r * r;
             }
+            return total(a);
+        };
+        const double r0 = r2();
+        for (int it = 0; it < A.max_sweeps && r0 > 0; it++) {
+            run(std::integral_constant<int, kSweep>(), L, L, w, 1);
+            if ((it & 7) == 7 && r2() <= A.reduce * A.reduce * r0) break;
         }
         double sz = 0;
         for (int p = t0; p < N; p += st) sz += double(L.z[(p / v.nx) * v.zp + p % v.nx]);
@@ -1103,33 +1256,201 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
         // (total() synchronises: every lane has read z before it changes)
         for (int p = t0; p < N; p += st) {
             const int i = p % v.nx, j = p / v.nx;
-            tput(L.la, L.z, i, j, L.z[j * v.zp + i] - mz);
+            tput(L, L.z, i, j, L.z[j * v.zp + i] - mz);
         }
         sync(w);
     };
     const int last = A.nlev - 1, ws = A.wave_from <= last ? A.wave_from : last + 1;
-    for (int l = 0; l < ws && l < last; l++) down(l, false);
+    constexpr std::integral_constant<int, kDown> down{};
+    constexpr std::integral_constant<int, kUp> up{};
+    Lv cur = top;  // the level at hand, read once on the way down and once up
+    for (int l = 0; l < ws && l < last; l++) {
+        const Lv next = lvl(l + 1);
+        run(down, cur, next, false, A.nu1);
+        cur = next;
+    }
     if (ws <= last) {
         if (tid < 64) {
-            for (int l = ws; l < last; l++) down(l, true);
-            coarsest(true);
-            for (int l = last - 1; l >= ws; l--) up(l, true);
+            for (int l = ws; l < last; l++) {
+                const Lv next = lvl(l + 1);
+                run(down, cur, next, true, A.nu1);
+                cur = next;
+            }
+            coarsest(cur, true);
+            for (int l = last - 1; l >= ws; l--) {
+                const Lv next = lvl(l);
+                run(up, next, cur, true, A.nu2);
+                cur = next;
+            }
         }
         __syncthreads();
     } else {
-        coarsest(false);
+        coarsest(cur, false);
     }
-    for (int l = (ws < last ? ws : last) - 1; l >= 0; l--) up(l, false);
+    const int from = (ws < last ? ws : last) - 1;
+    cur = lvl(from + 1);
+    for (int l = from; l >= 0; l--) {
+        const Lv next = lvl(l);
+        run(up, next, cur, false, A.nu2);
+        cur = next;
+    }
     {
         // the top level's iterate back, with its periodic ring mirrors
-        const TailLev &v = A.lv[0];
+        const TailLev &v = top.v;
         T *gz = (T *)A.z_top;
         const LevelArgs ga{v.nx, v.ny, A.top_pitch, A.top_pitch, v.kx, v.ky, px, py};
         for (int p = tid; p < v.nx * v.ny; p += nt) {
             const int i = p % v.nx, j = p / v.nx;
-            tput(ga, gz, i, j, arr(0, 0)[j * v.zp + i]);
+            const T z = top.z[j * v.zp + i];
+            if (PER) put_z(ga, gz, i, j, z);
+            else gz[j * A.top_pitch + i] = z;
         }
     }
+}
+
+// ---- the tail's coefficients: every level below its top one coarsened from
+// the one above (k_mac_coef_coarsen, k_fem_coef_coarsen), and the coarsest
+// level's matrix factored, in one workgroup: a launch instead of one per
+// level, and a factorisation per change of the coefficients instead of one
+// per V-cycle. The levels' FP64 arrays c1, c2 (and single-precision copies)
+// are laid out as k_tail holds them in LDS. A chain of a few dependent steps
+// per level, so all of them run in LDS between one read and one write of the
+// arrays: 8.7 us with the factors against five launches of 2.1 to 2.5 us for
+// the coefficients alone.
+struct TailCoefs {
+    TailArgs A;
+    int kind;
+    int direct;                // whether the coarsest level is factored
+    int copy;                  // all levels are there: only single-precision copies and factors
+    double *c1, *c2, *lu;
+    float *c1f, *c2f, *luf;    // null: no single-precision copies
+};
+constexpr int kTailCoefThreads = 512;
+// Entry (r, c) of the coarsest level's matrix (k_tail's `direct`: point 0 left
+// out of a pure-Neumann level), the terms added in the order of the stencil's.
+template <class T>
+__device__ __forceinline__ T tail_entry(const TailCoefs &C, const TailLev &v, const double *c1, const double *c2, int r,
+                                        int c) {
+    const TailArgs &A = C.A;
+    const int o = A.sing ? 1 : 0, N = v.nx * v.ny, p = r + o;
+    if (p >= N || c + o >= N) return T(0);
+    const int i = p % v.nx, j = p / v.nx, q = v.off + (j + 1) * v.zp + i + 1;
+    T s = 0;
+    auto put = [&](int di, int dj, T a) {
+        int ii = i + di, jj = j + dj;
+        if (A.px) ii = wrap_idx(ii, v.nx);
+        if (A.py) jj = wrap_idx(jj, v.ny);
+        if (ii < 0 || ii >= v.nx || jj < 0 || jj >= v.ny) return;
+        if (jj * v.nx + ii == c + o) s += a;
+    };
+    if (C.kind == kMAC) {
+        const T kx = T(v.kx), ky = T(v.ky);
+        const T wl = T(c1[q]), wr = T(c1[q + 1]), sd = T(c2[q]), su = T(c2[q + v.zp]);
+        put(0, 0, -(kx * (wl + wr) + ky * (sd + su)));
+        put(-1, 0, kx * wl);
+        put(1, 0, kx * wr);
+        put(0, -1, ky * sd);
+        put(0, 1, ky * su);
+    } else {
+        const FemC kk = A.k;
+        const T kdl = T(c1[q - v.zp - 1]), kdr = T(c1[q - v.zp]), kul = T(c1[q - 1]), kur = T(c1[q]);
+        put(0, 0, T(kk.fm) * (kdl + kdr + kul + kur));
+        put(-1, -1, T(kk.fc) * kdl);
+        put(1, -1, T(kk.fc) * kdr);
+        put(-1, 1, T(kk.fc) * kul);
+        put(1, 1, T(kk.fc) * kur);
+        put(0, -1, T(kk.hey) * (kdl + kdr));
+        put(0, 1, T(kk.hey) * (kul + kur));
+        put(-1, 0, T(kk.hex) * (kdl + kul));
+        put(1, 0, T(kk.hex) * (kdr + kur));
+    }
+    return s;
+}
+__global__ __launch_bounds__(kTailCoefThreads) void k_tail_coefs(TailCoefs C) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ double md[2][kTailDirect][kTailDirect + 1];
+    __shared__ float mf[2][kTailDirect][kTailDirect + 1];
+    const TailArgs &A = C.A;
+    const int tid = threadIdx.x, nt = kTailCoefThreads;
+    double *c1 = (double *)smem, *c2 = c1 + A.total;
+    const bool mac = C.kind == kMAC;
+    {
+        const int have = C.copy || A.nlev == 1 ? A.total : A.lv[1].off;  // the top level comes first
+        for (int p = tid; p < A.total; p += nt) {
+            c1[p] = p < have ? C.c1[p] : 0.0;
+            if (mac) c2[p] = p < have ? C.c2[p] : 0.0;
+        }
+    }
+    __syncthreads();
+    for (int l = 0; !C.copy && l + 1 < A.nlev; l++) {
+        const TailLev f = A.lv[l], c = A.lv[l + 1];
+        const int fo = f.off + f.zp + 1, co = c.off + c.zp + 1;
+        // coarse rows of (nx + 1) faces, or of nx (periodic, zero-pressure)
+        // or nx - 1 cells
+        const int W = mac ? c.nx + 1 : c.nx - ((A.px || A.dr) ? 0 : 1), H = mac ? c.ny + 1 : c.ny - (A.py ? 0 : 1);
+        for (int p = tid; p < W * H; p += nt) {
+            const int J = p / W, I = p - J * W, q = fo + 2 * J * f.zp + 2 * I, t = co + J * c.zp + I;
+            if (mac) {
+                if (J < c.ny) c1[t] = 0.5 * (c1[q] + c1[q + f.zp]);
+                if (I < c.nx) c2[t] = 0.5 * (c2[q] + c2[q + 1]);
+            } else {
+                const LevelArgs la{c.nx, c.ny, c.zp, c.zp, 0, 0, A.px, A.py, 0};
+                put_z(la, c1 + co, I, J, 0.25 * (c1[q] + c1[q + 1] + c1[q + f.zp] + c1[q + f.zp + 1]));
+            }
+        }
+        __syncthreads();
+    }
+    for (int p = (C.copy || A.nlev == 1 ? 0 : A.lv[1].off) + tid; p < A.total; p += nt) {
+        if (!C.copy) {
+            C.c1[p] = c1[p];
+            if (mac) C.c2[p] = c2[p];
+        }
+        if (C.c1f) {
+            C.c1f[p] = float(c1[p]);
+            if (mac) C.c2f[p] = float(c2[p]);
+        }
+    }
+    if (!C.direct) return;
+    // The factors, without pivoting, entry (r, c) in thread 16 r + c (the
+    // second half of the workgroup in single precision); not valid when a
+    // pivot is zero, not finite or of another sign than the first.
+    const TailLev v = A.lv[A.nlev - 1];
+    const int n = v.nx * v.ny - (A.sing ? 1 : 0);
+    const bool dbl = tid < kTailDirect * kTailDirect;
+    const int r = (tid & (kTailDirect * kTailDirect - 1)) / kTailDirect, c = tid % kTailDirect;
+    auto factor = [&](auto (&m)[2][kTailDirect][kTailDirect + 1], auto a, int k, bool &ok, auto s0) {
+        using T = decltype(a);
+        const T piv = m[k & 1][k][k], up = m[k & 1][k][c], left = m[k & 1][r][k];
+        if (!(piv == piv) || piv == T(0) || (piv > T(0)) != (s0 > T(0)) || !(piv * T(0) == T(0))) ok = false;
+        if (r > k) {
+            const T f = left / piv;
+            if (c == k) a = f;
+            else if (c > k) a -= f * up;
+        }
+        m[(k + 1) & 1][r][c] = a;
+        return a;
+    };
+    double ad = 0;
+    float af = 0;
+    if (dbl) md[0][r][c] = ad = tail_entry<double>(C, v, c1, c2, r, c);
+    else mf[0][r][c] = af = tail_entry<float>(C, v, c1, c2, r, c);
+    __syncthreads();
+    const double sd = md[0][0][0];
+    const float sf = mf[0][0][0];
+    bool ok = true;
+    for (int k = 0; k < n; k++) {
+        if (dbl) ad = factor(md, ad, k, ok, sd);
+        else af = factor(mf, af, k, ok, sf);
+        __syncthreads();
+    }
+    auto write = [&](auto *out, auto a) {
+        using T = decltype(a);
+        out[r * kTailDirect + c] = a;
+        if (r == c) out[kTailDirect * kTailDirect + r] = r < n ? T(1) / a : T(1);
+        if (r == 0 && c == 0) out[kTailLu - 1] = ok ? T(1) : T(0);
+    };
+    if (dbl) write(C.lu, ad);
+    else if (C.luf && C.c1f) write(C.luf, af);
 }
 
 // ------------------------------------------------------ coefficient setup
@@ -1643,35 +1964,77 @@ static size_t tail_start(const std::vector<MgLevel> &L) {
     return t;
 }
 
-template <class T>
-static TailArgs tail_args(const std::vector<MgLevel> &L, size_t t, MgKind kind, FemC k, int nu1, int nu2, bool f32,
-                          size_t *shmem) {
+// The tail's levels, from level t down: their LDS layout and parameters.
+static TailArgs tail_levels(const std::vector<MgLevel> &L, size_t t, MgKind kind, int nu1, int nu2) {
     TailArgs A{};
-    A.kind = kind; A.nlev = (int)(L.size() - t); A.nu1 = nu1; A.nu2 = nu2; A.k = k;
+    A.nlev = (int)(L.size() - t); A.nu1 = nu1; A.nu2 = nu2;
     A.px = L[t].px; A.py = L[t].py; A.dr = L[t].dr; A.sing = L[t].dr ? 0 : 1;
     int off = 0;
     A.wave_from = A.nlev;
     for (int q = 0; q < A.nlev; q++) {
         const MgLevel &v = L[t + q];
         TailLev &d = A.lv[q];
-        d.nx = v.nx; d.ny = v.ny; d.zp = v.nx + 2; d.off = off; d.gcp = v.cp; d.kx = v.kx; d.ky = v.ky;
-        const unsigned ha = (unsigned)(v.nx + 1) / 2;
-        d.mag = ((1u << 20) + ha - 1) / ha;
-        if (A.wave_from == A.nlev && (long long)v.nx * v.ny <= kTailWavePts) A.wave_from = q;
-        if (kind == kMAC) { d.c1 = f32 ? (const void *)v.fwf : v.fw; d.c2 = f32 ? (const void *)v.fsf : v.fs; }
-        else { d.c1 = f32 ? (const void *)v.kcf : v.kc; d.c2 = nullptr; }
+        d.nx = v.nx; d.ny = v.ny; d.zp = v.nx + 2; d.off = off; d.kx = v.kx; d.ky = v.ky;
+        d.ha = (v.nx + 1) / 2;
+        d.ng = d.ha * (kind == kMAC ? v.ny : (v.ny + 1) / 2);
+        d.mag = ((1u << 20) + d.ha - 1) / d.ha;
+        if (A.wave_from == A.nlev && d.ng <= kTailWaveGroups) A.wave_from = q;
         off += (v.nx + 2) * (v.ny + 2);
     }
     A.total = off;
-    A.z_top = f32 ? (void *)L[t].zf : (void *)L[t].z;
-    A.b_top = f32 ? (const void *)L[t].bf : (const void *)L[t].b;
-    A.top_pitch = L[t].pitch;
-    A.reduce = f32 ? 1e-5 : 1e-6;
     A.max_sweeps = 20000;
-    *shmem = (size_t)kTailArrays * off * sizeof(T);
     return A;
 }
 
+// One tail cycle in double or single precision.
+template <class T>
+int Multigrid::tail_cycle(size_t t) {
+    constexpr bool f32 = sizeof(T) == sizeof(float);
+    TailArgs A = tail_levels(L, t, kind_, nu1, nu2);
+    A.k = fem_consts(L[t].hx, L[t].hy);
+    A.z_top = f32 ? (void *)L[t].zf : (void *)L[t].z;
+    A.b_top = f32 ? (const void *)L[t].bf : (const void *)L[t].b;
+    A.c1 = f32 ? (const void *)tail_cf_[0] : tail_c_[0];
+    A.c2 = f32 ? (const void *)tail_cf_[1] : tail_c_[1];
+    A.lu = f32 ? (const void *)tail_luf_ : tail_lu_;
+    A.top_pitch = L[t].pitch;
+    A.reduce = f32 ? 1e-5 : 1e-6;
+    // a group a thread on the top level, two at most (256 threads with two
+    // groups each at 32^2 points made a cycle 1.9 us longer), and no more
+    // threads: each further wavefront lengthens every barrier
+    int threads = 256;
+    if (A.wave_from > 0) threads = std::max(threads, std::min(kTailThreads, (A.lv[0].ng + 63) / 64 * 64));
+    const size_t sh = (size_t)kTailArrays * A.total * sizeof(T);
+    const bool per = A.px || A.py;
+    if (kind_ == kMAC) {
+        if (per) k_tail<T, kMAC, true><<<1, threads, sh, s_>>>(A);
+        else k_tail<T, kMAC, false><<<1, threads, sh, s_>>>(A);
+    } else {
+        if (per) k_tail<T, kFEM, true><<<1, threads, sh, s_>>>(A);
+        else k_tail<T, kFEM, false><<<1, threads, sh, s_>>>(A);
+    }
+    KCHECK();
+    return 0;
+}
+
+// The tail's coefficients below its top level and the coarsest level's
+// factors, from the top level's coefficients; copy: only the
+// single-precision copies of the FP64 ones and their factors.
+int Multigrid::tail_coefs(bool f32, bool copy) {
+    if (tail_ >= L.size()) return 0;
+    TailCoefs C{};
+    const MgLevel &t = L[tail_];
+    C.A = tail_levels(L, tail_, kind_, nu1, nu2);
+    C.A.k = fem_consts(t.hx, t.hy);
+    C.kind = kind_;
+    C.direct = tail_lu_ != nullptr;
+    C.copy = copy;
+    C.c1 = tail_c_[0]; C.c2 = tail_c_[1]; C.lu = tail_lu_;
+    if (f32 || copy) { C.c1f = tail_cf_[0]; C.c2f = tail_cf_[1]; C.luf = tail_luf_; }
+    k_tail_coefs<<<1, kTailCoefThreads, (kind_ == kMAC ? 2 : 1) * (size_t)C.A.total * sizeof(double), s_>>>(C);
+    KCHECK();
+    return 0;
+}
 
 Multigrid::~Multigrid() {
     for (auto &g : graph_exec_)
@@ -1799,13 +2162,6 @@ int Multigrid::init(MgKind kind, int m, int n, double dx, double dy, hipStream_t
         int rc;
         if ((rc = dalloc(l.z)) || (rc = dalloc(l.z2)) || (rc = dalloc(l.b)) || (rc = dalloc(l.r))) return rc;
         if ((rc = falloc(l.zf)) || (rc = falloc(l.zf2)) || (rc = falloc(l.bf)) || (rc = falloc(l.rf))) return rc;
-        if (kind == kMAC) {
-            if ((rc = dalloc(l.fw)) || (rc = dalloc(l.fs))) return rc;
-            if ((rc = falloc(l.fwf)) || (rc = falloc(l.fsf))) return rc;
-        } else {
-            if ((rc = dalloc(l.kc))) return rc;
-            if ((rc = falloc(l.kcf))) return rc;
-        }
         l.hx = hx; l.hy = hy;
         L.push_back(l);
         if (kind == kFEM && !px && !py && !dr && L.size() == 1 && nx >= 5 && ny >= 5 && (nx % 2 == 0 || ny % 2 == 0)) {
@@ -1867,7 +2223,7 @@ int Multigrid::init(MgKind kind, int m, int n, double dx, double dy, hipStream_t
     d_red = (double *)q;
     HIP_CHECK(hipHostMalloc((void **)&h_red, 8 * sizeof(double), hipHostMallocDefault));
     tail_ = tail_start(L);
-    // the tail kernel divides colour indices k < ha * rows by ha = (nx+1)/2
+    // the tail kernel divides group indices k < ha * rows by ha = (nx+1)/2
     // as (k * ceil(2^20/ha)) >> 20: check it is exact on every tail level
     for (size_t l = tail_; l < L.size(); l++) {
         const unsigned ha = (unsigned)(L[l].nx + 1) / 2, mag = ((1u << 20) + ha - 1) / ha;
@@ -1876,16 +2232,58 @@ int Multigrid::init(MgKind kind, int m, int n, double dx, double dy, hipStream_t
                 return INCRMT_ERR_GRID;
     }
     if (resampled_ && tail_ == 0) tail_ = 1;  // the tail's transfers assume nested levels
+    if (int rc = alloc_coefs()) return rc;
     if (int rc = set_irho_host(nullptr)) return rc;
     return autotune();
 }
 
 
+// Coefficient arrays: a level's own above the tail; the tail's levels one
+// behind the other, each with the pitch nx + 2 that the tail kernel gives it
+// in LDS, so that it loads them all as one flat range.
+int Multigrid::alloc_coefs() {
+    auto zeroed = [&](auto *&p, size_t n) -> int {
+        void *q;
+        HIP_CHECK(hipMalloc(&q, n * sizeof(*p)));
+        HIP_CHECK(memset_sync(q, 0, n * sizeof(*p), s_));
+        allocs.push_back(q);
+        p = (std::remove_reference_t<decltype(p)>)q;
+        return 0;
+    };
+    size_t total = 0;
+    for (size_t l = tail_; l < L.size(); l++) total += (size_t)(L[l].nx + 2) * (L[l].ny + 2);
+    const int arrays = kind_ == kMAC ? 2 : 1;
+    int rc;
+    for (int a = 0; a < arrays && total; a++)
+        if ((rc = zeroed(tail_c_[a], total)) || (rc = zeroed(tail_cf_[a], total))) return rc;
+    size_t off = 0;
+    for (size_t l = 0; l < L.size(); l++) {
+        MgLevel &v = L[l];
+        double *c[2] = {nullptr, nullptr};
+        float *cf[2] = {nullptr, nullptr};
+        if (l >= tail_) v.cp = v.nx + 2;
+        const size_t len = (size_t)(v.ny + 2) * v.cp;
+        for (int a = 0; a < arrays; a++) {
+            if (l >= tail_) { c[a] = tail_c_[a] + off; cf[a] = tail_cf_[a] + off; }
+            else if ((rc = zeroed(c[a], len + 64)) || (rc = zeroed(cf[a], len + 64))) return rc;
+            c[a] += v.cp + 1;
+            cf[a] += v.cp + 1;
+        }
+        if (l >= tail_) off += len;
+        if (kind_ == kMAC) { v.fw = c[0]; v.fs = c[1]; v.fwf = cf[0]; v.fsf = cf[1]; }
+        else { v.kc = c[0]; v.kcf = cf[0]; }
+    }
+    const long long last = (long long)L.back().nx * L.back().ny;
+    if (total && last > 1 && last <= kTailDirect)
+        if ((rc = zeroed(tail_lu_, kTailLu)) || (rc = zeroed(tail_luf_, kTailLu))) return rc;
+    return 0;
+}
+
 int Multigrid::coarsen_coefs(bool f32) {
     // f32: the caller wrote level 0's single-precision copies with its
     // coefficients; every coarse level writes its copies too
     if (resampled_) f32 = false;
-    for (size_t l = 0; l + 1 < L.size(); l++) {
+    for (size_t l = 0; l + 1 < L.size() && l < tail_; l++) {
         const MgLevel &f = L[l];
         MgLevel &c = L[l + 1];
         if (kind_ == kMAC && l == 0 && rs_per_) {
@@ -1909,23 +2307,24 @@ int Multigrid::coarsen_coefs(bool f32) {
     }
     // otherwise the single-precision copies are made when a mixed solve needs them
     f32_stale_ = !f32;
-    return 0;
+    return tail_coefs(f32, false);
 }
 
 int Multigrid::make_f32_coefs() {
     f32_stale_ = false;
-    for (auto &l : L) {
-        const long long len = (long long)(l.ny + 2) * l.pitch;
+    for (size_t q = 0; q < L.size() && q < tail_; q++) {
+        const MgLevel &l = L[q];
+        const long long len = (long long)(l.ny + 2) * l.cp;
         const int nb = (int)((len + 255) / 256);
         if (kind_ == kMAC) {
-            k_to_f32<<<nb, 256, 0, s_>>>(l.fw - l.pitch - 1, l.fwf - l.pitch - 1, len);
-            k_to_f32<<<nb, 256, 0, s_>>>(l.fs - l.pitch - 1, l.fsf - l.pitch - 1, len);
+            k_to_f32<<<nb, 256, 0, s_>>>(l.fw - l.cp - 1, l.fwf - l.cp - 1, len);
+            k_to_f32<<<nb, 256, 0, s_>>>(l.fs - l.cp - 1, l.fsf - l.cp - 1, len);
         } else {
-            k_to_f32<<<nb, 256, 0, s_>>>(l.kc - l.pitch - 1, l.kcf - l.pitch - 1, len);
+            k_to_f32<<<nb, 256, 0, s_>>>(l.kc - l.cp - 1, l.kcf - l.cp - 1, len);
         }
         KCHECK();
     }
-    return 0;
+    return tail_coefs(true, true);
 }
 
 int Multigrid::set_density(const Grid &g, const double *rho) {
@@ -1948,10 +2347,12 @@ int Multigrid::wrap_coefs(size_t l, bool f32) {
     const MgLevel &v = L[l];
     if (kind_ != kFEM || !(v.px || v.py)) return 0;
     const int n = 2 * (v.nx + 2) + 2 * (v.ny + 2);
-    k_wrap_ring<double><<<(n + 255) / 256, 256, 0, s_>>>(args_of(v), v.kc);
+    LevelArgs a = args_of(v);
+    a.zp = a.cp;
+    k_wrap_ring<double><<<(n + 255) / 256, 256, 0, s_>>>(a, v.kc);
     KCHECK();
     if (f32) {
-        k_wrap_ring<float><<<(n + 255) / 256, 256, 0, s_>>>(args_of(v), v.kcf);
+        k_wrap_ring<float><<<(n + 255) / 256, 256, 0, s_>>>(a, v.kcf);
         KCHECK();
     }
     return 0;
@@ -1969,8 +2370,8 @@ int Multigrid::wrap_fine(double *z) {
 int Multigrid::set_irho_host(const double *irho) {
     MgLevel &f = L[0];
     const int nx = f.nx, ny = f.ny;
-    std::vector<double> h((size_t)(ny + 2) * f.pitch, 0.0);
-    auto at = [&](int i, int j) -> double & { return h[(size_t)(j + 1) * f.pitch + i + 1]; };
+    std::vector<double> h((size_t)(ny + 2) * f.cp, 0.0);
+    auto at = [&](int i, int j) -> double & { return h[(size_t)(j + 1) * f.cp + i + 1]; };
     const bool px = f.px, py = f.py;
     if (kind_ == kMAC) {
         // fw from the left-edge entries, walls zero (mgs_mac.hh:64-102); a
@@ -1982,13 +2383,13 @@ int Multigrid::set_irho_host(const double *irho) {
             if (px) at(nx, j) = irho ? irho[2 * mn + j] : 1.0;
             if (f.dr) at(nx, j) = 2 * (irho ? irho[2 * mn + j] : 1.0);
         }
-        HIP_CHECK(hipMemcpy(f.fw - f.pitch - 1, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+        HIP_CHECK(hipMemcpy(f.fw - f.cp - 1, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
         std::fill(h.begin(), h.end(), 0.0);
         for (int j = py ? 0 : 1; j < ny; j++)
             for (int i = 0; i < nx; i++) at(i, j) = irho ? irho[2 * (j * nx + i) + 1] : 1.0;
         if (py)
             for (int i = 0; i < nx; i++) at(i, ny) = irho ? irho[2 * mn + ny + i] : 1.0;
-        HIP_CHECK(hipMemcpy(f.fs - f.pitch - 1, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+        HIP_CHECK(hipMemcpy(f.fs - f.cp - 1, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
     } else {
         // cell (i,j) weight = irho of its upper-right node (mgs_fem.hh:99-106),
         // node nx being node 0 along a periodic direction; with a
@@ -1997,7 +2398,7 @@ int Multigrid::set_irho_host(const double *irho) {
         for (int j = 0; j < ny - (py ? 0 : 1); j++)
             for (int i = 0; i < nx - ((px || f.dr) ? 0 : 1); i++)
                 at(i, j) = irho ? irho[(size_t)((j + 1) % ny) * rl + (i + 1) % rl] : 1.0;
-        HIP_CHECK(hipMemcpy(f.kc - f.pitch - 1, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+        HIP_CHECK(hipMemcpy(f.kc - f.cp - 1, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
         if (int rc = wrap_coefs(0)) return rc;
     }
     return coarsen_coefs();
@@ -2405,14 +2806,7 @@ int Multigrid::smooth_fine(int sweeps, bool fp32) { return fp32 ? smooth_f(0, sw
 int Multigrid::vcycle(size_t l) {
     const MgLevel &f = L[l];
     const FemC k = fem_consts(f.hx, f.hy);
-    if (l == tail_) {
-        size_t sh;
-        const TailArgs A = tail_args<double>(L, l, kind_, k, nu1, nu2, false, &sh);
-        if (A.px || A.py) k_tail<double, true><<<1, kTailThreads, sh, s_>>>(A);
-        else k_tail<double, false><<<1, kTailThreads, sh, s_>>>(A);
-        KCHECK();
-        return 0;
-    }
+    if (l == tail_) return tail_cycle<double>(l);
     if (l + 1 == L.size()) {
         k_coarse_solve<double><<<1, 256, 0, s_>>>(kind_, args_of(f), k, f.z, f.b, f.fw, f.fs, f.kc, 1e-6, 20000,
                                                   singular());
@@ -2470,14 +2864,7 @@ int Multigrid::vcycle(size_t l) {
 int Multigrid::vcycle_f(size_t l) {
     const MgLevel &f = L[l];
     const FemC k = fem_consts(f.hx, f.hy);
-    if (l == tail_) {
-        size_t sh;
-        const TailArgs A = tail_args<float>(L, l, kind_, k, nu1, nu2, true, &sh);
-        if (A.px || A.py) k_tail<float, true><<<1, kTailThreads, sh, s_>>>(A);
-        else k_tail<float, false><<<1, kTailThreads, sh, s_>>>(A);
-        KCHECK();
-        return 0;
-    }
+    if (l == tail_) return tail_cycle<float>(l);
     if (l + 1 == L.size()) {
         k_coarse_solve<float><<<1, 256, 0, s_>>>(kind_, args_of(f), k, f.zf, f.bf, f.fwf, f.fsf, f.kcf, 1e-5, 20000,
                                                  singular());
