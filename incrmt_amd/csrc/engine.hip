@@ -15,6 +15,7 @@
 #include <limits>
 #include <atomic>
 #include <chrono>
+#include "hostcopy.hh"
 #include "step.hh"
 #include "mg.hh"
 #include "levelset.hh"
@@ -187,6 +188,7 @@ struct FluidEngine {
         pev_used = 0;
         return 0;
     }
+    HostCopy copy;        // field downloads and uploads
     int launch_req = -1;  // V-cycle issue mode asked for (-1: the solvers' default by size)
     TracerSet tr;
 
@@ -705,6 +707,7 @@ struct incrmt_mg {
     hipStream_t s = nullptr;
     double *x = nullptr, *y = nullptr;
     double *bkeep = nullptr;  // the last solve's right-hand side (timed solves)
+    HostCopy copy;
     // host row length: the solver's nx, plus the fixed node column of a FEM
     // system with zero pressure on the right edge (read as zero, written
     // as zero)
@@ -723,14 +726,7 @@ namespace {
 int copy_field(FluidEngine &e, double *dev, double *host, bool down) {
     const Grid &g = e.g;
     double *d0 = dev + g.ls(0, 0);
-    if (down)
-        HIP_CHECK(hipMemcpy2DAsync(host, g.ml * sizeof(double), d0, g.P * sizeof(double), g.ml * sizeof(double), g.nl,
-                                   hipMemcpyDeviceToHost, e.s));
-    else
-        HIP_CHECK(hipMemcpy2DAsync(d0, g.P * sizeof(double), host, g.ml * sizeof(double), g.ml * sizeof(double), g.nl,
-                                   hipMemcpyHostToDevice, e.s));
-    HIP_CHECK(hipStreamSynchronize(e.s));
-    return 0;
+    return down ? e.copy.down(e.s, d0, g.P, g.ml, g.ml, g.nl, host) : e.copy.up(e.s, d0, g.P, g.ml, g.ml, g.nl, host);
 }
 
 double *field_ptr(FluidEngine &e, const std::string &nm, int k, bool &is_int) {
@@ -989,11 +985,7 @@ int incrmt_fluid_download(incrmt_fluid *f, const char *name, int obj, double *ho
     FluidEngine &e = f->e;
     HIP_CHECK(hipStreamSynchronize(e.s));
     if (!is_int) return copy_field(e, p, host, true);
-    std::vector<int> tmp(e.g.N);
-    HIP_CHECK(hipMemcpy(tmp.data(), p, e.g.N * sizeof(int), hipMemcpyDeviceToHost));
-    for (int J = 0; J < e.g.nl; J++)
-        for (int I = 0; I < e.g.ml; I++) host[J * e.g.ml + I] = tmp[e.g.ls(I, J)];
-    return 0;
+    return e.copy.down(e.s, (const int *)p + e.g.ls(0, 0), e.g.P, e.g.ml, e.g.ml, e.g.nl, host);
 }
 
 int incrmt_fluid_upload(incrmt_fluid *f, const char *name, int obj, const double *host) {
@@ -1615,19 +1607,10 @@ int incrmt_mg_set_irho(incrmt_mg *h, const double *irho) {
 }
 
 static int mg_copy(incrmt_mg *h, double *dev, const double *host_in, double *host_out) {
+    // (the fixed column, past the level's nx, reads as zero)
     const MgLevel &l = h->mg.fine();
-    const size_t hp = (size_t)h->hm * sizeof(double);
-    if (host_in)
-        HIP_CHECK(hipMemcpy2DAsync(dev, l.pitch * sizeof(double), host_in, hp, l.nx * sizeof(double), l.ny,
-                                   hipMemcpyHostToDevice, h->s));
-    else
-        HIP_CHECK(hipMemcpy2DAsync(host_out, hp, dev, l.pitch * sizeof(double), l.nx * sizeof(double), l.ny,
-                                   hipMemcpyDeviceToHost, h->s));
-    HIP_CHECK(hipStreamSynchronize(h->s));
-    if (host_out)
-        for (int j = 0; j < l.ny; j++)
-            for (int i = l.nx; i < h->hm; i++) host_out[(size_t)j * h->hm + i] = 0;  // the fixed column
-    return 0;
+    return host_in ? h->copy.up(h->s, dev, l.pitch, h->hm, l.nx, l.ny, host_in)
+                   : h->copy.down(h->s, dev, l.pitch, h->hm, l.nx, l.ny, host_out);
 }
 
 int incrmt_mg_solve(incrmt_mg *h, const double *b, double *z, double rel_tol, int max_cycles, int precision,
@@ -1782,21 +1765,10 @@ struct LsStandalone {
         a.st = (int *)q;
         return ls_alloc(g, w, s);
     }
-    int put(double *dev, const double *host) {
-        HIP_CHECK(hipMemcpy2D(dev + g.ls(0, 0), g.P * sizeof(double), host, g.ml * sizeof(double),
-                              g.ml * sizeof(double), g.nl, hipMemcpyHostToDevice));
-        return 0;
-    }
-    int get(const double *dev, double *host) {
-        HIP_CHECK(hipMemcpy2D(host, g.ml * sizeof(double), dev + g.ls(0, 0), g.P * sizeof(double),
-                              g.ml * sizeof(double), g.nl, hipMemcpyDeviceToHost));
-        return 0;
-    }
-    int get_status(int *host) {
-        HIP_CHECK(hipMemcpy2D(host, g.ml * sizeof(int), a.st + g.ls(0, 0), g.P * sizeof(int), g.ml * sizeof(int),
-                              g.nl, hipMemcpyDeviceToHost));
-        return 0;
-    }
+    HostCopy copy;
+    int put(double *dev, const double *host) { return copy.up(s, dev + g.ls(0, 0), g.P, g.ml, g.ml, g.nl, host); }
+    int get(const double *dev, double *host) { return copy.down(s, dev + g.ls(0, 0), g.P, g.ml, g.ml, g.nl, host); }
+    int get_status(int *host) { return copy.down(s, (const int *)a.st + g.ls(0, 0), g.P, g.ml, g.ml, g.nl, host); }
 };
 int ls_args_ok(int m, int n, double dx, double dy, double pd, double pu) {
     if (m < 8 || n < 8 || !(dx > 0) || !(dy > 0) || !(pd < 0) || !(pu > 0))
