@@ -250,9 +250,10 @@ class Multigrid {
     int vcycle_f(size_t l);
     int coarsen_coefs(bool f32 = false);
     int reduce_norms(double *out3);  // ||b||^2, ||r||^2, sum b of level 0
-    int reduce_dev();                // the same into d_red, no host copy
+    int reduce_dev(double *host = nullptr);  // the same into d_red (and pinned host memory)
+    int mixed_step(bool add, double *out3);
     template <class Cycle>
-    int solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle);
+    int solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle, bool fused = false);
     int predict_ = 0;                // V-cycles run before the first residual check
     double *zprev_ = nullptr;        // the solution before the last one (extrapolation)
     bool f32_stale_ = true;          // coefficient copies for the FP32 cycle out of date

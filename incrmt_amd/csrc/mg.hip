@@ -1592,7 +1592,7 @@ __global__ void k_norms(int kind, LevelArgs a, FemC k, const double *z, const do
     }
 }
 // Fixed-order sum of the partials into out[0..2].
-__global__ void k_sum_partials(const double *part, int nb, double *out) {
+__global__ void k_sum_partials(const double *part, int nb, double *out, double *host = nullptr) {
     __shared__ double s[3][kRedThreads];
     for (int k = 0; k < 3; k++) {
         double v = 0;
@@ -1606,7 +1606,48 @@ __global__ void k_sum_partials(const double *part, int nb, double *out) {
         __syncthreads();
     }
     if (threadIdx.x == 0)
-        for (int k = 0; k < 3; k++) out[k] = s[k][0];
+        for (int k = 0; k < 3; k++) {
+            out[k] = s[k][0];
+            if (host) host[k] = s[k][0];  // pinned memory: no copy behind the kernel
+        }
+}
+// The sums of z and b that k_norms forms of its right-hand side, by themselves
+// and in the same order: a mean needs neither the residual nor the
+// coefficients (z may be null).
+__global__ void k_sums(LevelArgs a, const double *z, const double *b, double *part) {
+    __shared__ double s1[kRedThreads], s2[kRedThreads];
+    double zs = 0, bs = 0;
+    const int N = a.nx * a.ny, S = gridDim.x * blockDim.x, di = S % a.nx, dj = S / a.nx;
+    const int p0 = blockIdx.x * blockDim.x + threadIdx.x;
+    int i = p0 % a.nx, j = p0 / a.nx;
+#pragma unroll 4
+    for (int p = p0; p < N; p += S) {
+        const int q = j * a.zp + i;
+        if (z) zs += z[q];
+        bs += b[q];
+        i += di;
+        j += dj;
+        if (i >= a.nx) { i -= a.nx; j++; }
+    }
+    s1[threadIdx.x] = zs; s2[threadIdx.x] = bs;
+    __syncthreads();
+    for (int w = kRedThreads / 2; w > 0; w >>= 1) {
+        if (threadIdx.x < w) {
+            s1[threadIdx.x] += s1[threadIdx.x + w];
+            s2[threadIdx.x] += s2[threadIdx.x + w];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        part[3 * blockIdx.x] = 0; part[3 * blockIdx.x + 1] = s1[0]; part[3 * blockIdx.x + 2] = s2[0];
+    }
+}
+__global__ void k_sub_means(LevelArgs a, double *z, double *b, const double *sums) {
+    const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y;
+    if (i >= a.nx || j >= a.ny) return;
+    const int q = j * a.zp + i;
+    if (z) z[q] -= sums[1] / (double(a.nx) * a.ny);
+    b[q] -= sums[2] / (double(a.nx) * a.ny);
 }
 __global__ void k_sub_mean(LevelArgs a, double *b, const double *sums) {
     const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y;
@@ -1760,6 +1801,81 @@ __global__ void k_copy_level(LevelArgs a, const double *z, double *zp) {
     const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y;
     if (i >= a.nx || j >= a.ny) return;
     zp[j * a.zp + i] = z[j * a.zp + i];
+}
+// The end of one mixed cycle and the start of the next in one pass, on a
+// walled level: z2 = z + e (e the single-precision correction; null: the
+// iterate stays where it is), the residual b - A z2 rounded into bf, and the
+// next correction's iterate cleared (zf2; a neighbour may still read e, so not
+// in e's place). Each neighbour's new value is formed again from z and e, with
+// k_add_f32's and k_residual_f32's expressions. Memory bound: 60 bytes a MAC
+// point in two passes become 52 in one, with the norms 92 in three passes 52
+// (FEM 52 and 76 become 44). At 1024^2 13.6 us MAC, 17.1 FEM, 16.4 and 20.0
+// with the norms; 24 steps of a fluid at 1024^2 70.1 -> 69.1 ms.
+template <int KIND>
+__device__ __forceinline__ double mixed_point(const LevelArgs &a, const FemC &k, const double *z, const float *e,
+                                              const double *b, const double *c1, const double *c2, double *z2, float *bf,
+                                              float *zf2, int q, int c, double &bq) {
+    auto Z = [&](int o) { return e ? z[q + o] + double(e[q + o]) : z[q + o]; };
+    const int zp = a.zp, cp = a.cp;
+    const double zc = Z(0);
+    double diag, off;
+    bq = b[q];
+    if (KIND == kMAC) {
+        const double wl = c1[c], wr = c1[c + 1], sd = c2[c], su = c2[c + cp];
+        diag = -(a.kx * (wl + wr) + a.ky * (sd + su));
+        off = a.kx * (wl * Z(-1) + wr * Z(1)) + a.ky * (sd * Z(-zp) + su * Z(zp));
+    } else {
+        const double kdl = c1[c - cp - 1], kdr = c1[c - cp], kul = c1[c - 1], kur = c1[c];
+        diag = k.fm * (kdl + kdr + kul + kur);
+        off = k.fc * (kdl * Z(-zp - 1) + kdr * Z(-zp + 1) + kul * Z(zp - 1) + kur * Z(zp + 1)) +
+              k.hey * ((kdl + kdr) * Z(-zp) + (kul + kur) * Z(zp)) + k.hex * ((kdl + kul) * Z(-1) + (kdr + kur) * Z(1));
+    }
+    const double r = bq - off - diag * zc;
+    bf[q] = float(r);
+    zf2[q] = 0;
+    if (e) z2[q] = zc;
+    return r;
+}
+template <int KIND>
+__global__ void k_mixed_step(LevelArgs a, FemC k, const double *z, const float *e, const double *b, const double *c1,
+                             const double *c2, double *z2, float *bf, float *zf2) {
+    const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y;
+    if (i >= a.nx || j >= a.ny) return;
+    double bq;
+    mixed_point<KIND>(a, k, z, e, b, c1, c2, z2, bf, zf2, j * a.zp + i, j * a.cp + i, bq);
+}
+// ... with the norms of a residual check, in k_norms' order
+template <int KIND>
+__global__ __launch_bounds__(kRedThreads) void k_mixed_check(LevelArgs a, FemC k, const double *z, const float *e,
+                                                             const double *b, const double *c1, const double *c2,
+                                                             double *z2, float *bf, float *zf2, double *part) {
+    __shared__ double s0[kRedThreads], s1[kRedThreads];
+    double bb = 0, rr = 0;
+    const int N = a.nx * a.ny, S = gridDim.x * blockDim.x, di = S % a.nx, dj = S / a.nx;
+    const int p0 = blockIdx.x * blockDim.x + threadIdx.x;
+    int i = p0 % a.nx, j = p0 / a.nx;
+#pragma unroll 4
+    for (int p = p0; p < N; p += S) {
+        double bq;
+        const double r = mixed_point<KIND>(a, k, z, e, b, c1, c2, z2, bf, zf2, j * a.zp + i, j * a.cp + i, bq);
+        bb += bq * bq;
+        rr += r * r;
+        i += di;
+        j += dj;
+        if (i >= a.nx) { i -= a.nx; j++; }
+    }
+    s0[threadIdx.x] = bb; s1[threadIdx.x] = rr;
+    __syncthreads();
+    for (int w = kRedThreads / 2; w > 0; w >>= 1) {
+        if (threadIdx.x < w) {
+            s0[threadIdx.x] += s0[threadIdx.x + w];
+            s1[threadIdx.x] += s1[threadIdx.x + w];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        part[3 * blockIdx.x] = s0[0]; part[3 * blockIdx.x + 1] = s1[0]; part[3 * blockIdx.x + 2] = 0;
+    }
 }
 __global__ void k_add_f32(LevelArgs a, double *z, const float *e) {
     const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y;
@@ -2937,21 +3053,57 @@ int Multigrid::vcycle_f(size_t l) {
     return smooth_f(l, nu2, true, true);
 }
 
-int Multigrid::reduce_dev() {
+int Multigrid::reduce_dev(double *host) {
     const MgLevel &f = L[0];
     k_norms<<<kRedBlocks, kRedThreads, 0, s_>>>(kind_, args_of(f), fem_consts(dx_, dy_), f.z, f.b, f.fw, f.fs, f.kc,
                                                 d_red + 8);
     KCHECK();
-    k_sum_partials<<<1, kRedThreads, 0, s_>>>(d_red + 8, kRedBlocks, d_red);
+    k_sum_partials<<<1, kRedThreads, 0, s_>>>(d_red + 8, kRedBlocks, d_red, host);
     KCHECK();
     return 0;
 }
 
 int Multigrid::reduce_norms(double *out3) {
-    if (int rc = reduce_dev()) return rc;
-    HIP_CHECK(hipMemcpyAsync(h_red, d_red, 3 * sizeof(double), hipMemcpyDeviceToHost, s_));
+    if (int rc = reduce_dev(h_red)) return rc;
     HIP_CHECK(hipStreamSynchronize(s_));
     for (int k = 0; k < 3; k++) out3[k] = h_red[k];
+    return 0;
+}
+
+// The residual of the iterate, after adding the last correction to it (add),
+// as the next mixed cycle's right-hand side; out3: with its norms, read back.
+// Current buffers change with every added correction, so a captured cycle
+// does not use it.
+int Multigrid::mixed_step(bool add, double *out3) {
+    MgLevel &f = L[0];
+    const FemC k = fem_consts(dx_, dy_);
+    const double *c1 = kind_ == kMAC ? f.fw : f.kc, *c2 = f.fs;
+    const float *e = add ? f.zf : nullptr;
+    float *clear = add ? f.zf2 : f.zf;
+    if (out3) {
+        if (kind_ == kMAC)
+            k_mixed_check<kMAC><<<kRedBlocks, kRedThreads, 0, s_>>>(args_of(f), k, f.z, e, f.b, c1, c2, f.z2, f.bf, clear,
+                                                                     d_red + 8);
+        else
+            k_mixed_check<kFEM><<<kRedBlocks, kRedThreads, 0, s_>>>(args_of(f), k, f.z, e, f.b, c1, c2, f.z2, f.bf, clear,
+                                                                     d_red + 8);
+        KCHECK();
+        k_sum_partials<<<1, kRedThreads, 0, s_>>>(d_red + 8, kRedBlocks, d_red, h_red);
+    } else if (kind_ == kMAC) {
+        k_mixed_step<kMAC><<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(args_of(f), k, f.z, e, f.b, c1, c2, f.z2, f.bf,
+                                                                        clear);
+    } else {
+        k_mixed_step<kFEM><<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(args_of(f), k, f.z, e, f.b, c1, c2, f.z2, f.bf,
+                                                                        clear);
+    }
+    KCHECK();
+    if (add) {
+        std::swap(f.z, f.z2);
+        std::swap(f.zf, f.zf2);
+    }
+    if (!out3) return 0;
+    HIP_CHECK(hipStreamSynchronize(s_));
+    for (int q = 0; q < 3; q++) out3[q] = h_red[q];
     return 0;
 }
 
@@ -2962,8 +3114,9 @@ int Multigrid::reduce_norms(double *out3) {
 // one, is run before the next residual check, so a solve costs two or three
 // host round trips instead of one per cycle; after that the residual is
 // checked after every cycle.
+// fused: mixed cycles whose ends and residuals go together (mixed_step)
 template <class Cycle>
-int Multigrid::solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle) {
+int Multigrid::solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle, bool fused) {
     const MgLevel &f = L[0];
     int rc;
     if ((rc = wrap_fine(f.z))) return rc;  // the iterate may come from outside
@@ -3045,24 +3198,19 @@ int Multigrid::solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle) 
             t0_ = t;
         }
     }
-    if (extrapolate && singular()) {
-        // an extrapolated start also carries the constant null-space part
-        // of the iterates forward, and the quadratic weights (3,-3,1 at
-        // equal steps) amplify any drift of it from solve to solve: the
-        // start is made mean-free (the caller uses only gradients and
-        // mean-free values, so the solution is unchanged)
-        k_norms<<<kRedBlocks, kRedThreads, 0, s_>>>(kind_, args_of(f), fem_consts(dx_, dy_), f.z, f.z, f.fw, f.fs,
-                                                    f.kc, d_red + 8);
+    if (singular()) {
+        // pure Neumann: only the mean-free part of b is solvable. An
+        // extrapolated start also carries the constant null-space part of
+        // the iterates forward, and the quadratic weights (3,-3,1 at equal
+        // steps) amplify any drift of it from solve to solve: such a start is
+        // made mean-free too (the caller uses only gradients and mean-free
+        // values, so the solution is unchanged)
+        double *z = extrapolate ? f.z : nullptr;
+        k_sums<<<kRedBlocks, kRedThreads, 0, s_>>>(args_of(f), z, f.b, d_red + 8);
         KCHECK();
         k_sum_partials<<<1, kRedThreads, 0, s_>>>(d_red + 8, kRedBlocks, d_red);
         KCHECK();
-        k_sub_mean<<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(args_of(f), f.z, d_red);
-        KCHECK();
-    }
-    if (singular()) {
-        // pure Neumann: only the mean-free part of b is solvable
-        if ((rc = reduce_dev())) return rc;
-        k_sub_mean<<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(args_of(f), f.b, d_red);
+        k_sub_means<<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(args_of(f), z, f.b, d_red);
         KCHECK();
     }
     // the learned start (mgs_base::initial_guess's hook, mgs_common.cc:33-66);
@@ -3092,13 +3240,21 @@ int Multigrid::solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle) 
     if ((learned || sample) && (rc = learned_start(learned))) return rc;
     if (measure) HIP_CHECK(hipEventRecord(cev_[1], s_));
     double nr[3];
-    if ((rc = reduce_norms(nr))) return rc;
+    if ((rc = fused ? mixed_step(false, nr) : reduce_norms(nr))) return rc;
     const double bn = std::sqrt(nr[0]);
     double rel = bn > 0 ? std::sqrt(nr[1]) / bn : 0;
     int cycles = 0;
     bool fallback = false;
     auto fp64_cycle = [&]() -> int { return run_cycle(0, [&]() { return vcycle(0); }); };
-    auto next = [&]() -> int { return fallback ? fp64_cycle() : cycle(); };
+    // one cycle, and a check of the residual behind it
+    auto next = [&](bool check) -> int {
+        if (fused) {
+            if (int e = vcycle_f(0)) return e;
+            return mixed_step(true, check ? nr : nullptr);
+        }
+        if (int e = fallback ? fp64_cycle() : cycle()) return e;
+        return check ? reduce_norms(nr) : 0;
+    };
     if (learned && rel > tol && bn > 0 && max_cycles > 0) {
         // one V-cycle, then the judgement in FP64: a learned start that has
         // not reached guess_tol is dropped for the quadratic start and plain
@@ -3131,15 +3287,13 @@ int Multigrid::solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle) 
     if (rel > tol && bn > 0 && predict_ > cycles) {
         const int ahead = predict_ < max_cycles ? predict_ : max_cycles;
         for (; cycles < ahead; cycles++)
-            if ((rc = next())) return rc;
-        if ((rc = reduce_norms(nr))) return rc;
+            if ((rc = next(cycles + 1 == ahead))) return rc;
         rel = std::sqrt(nr[1]) / bn;
     }
     while (rel > tol && bn > 0) {
         if (cycles >= max_cycles) break;
-        if ((rc = next())) return rc;
+        if ((rc = next(true))) return rc;
         cycles++;
-        if ((rc = reduce_norms(nr))) return rc;
         rel = std::sqrt(nr[1]) / bn;
     }
     if (cycles > 0) predict_ = cycles - 1;
@@ -3381,6 +3535,11 @@ int Multigrid::solve_mixed(double tol, int max_cycles, MgStats *st) {
         if (int rc = make_f32_coefs()) return rc;
     if (krylov && !f.px && !f.py && !f.dr && !resampled_) return solve_krylov(tol, max_cycles, st);
     const FemC k = fem_consts(dx_, dy_);
+    // The update and the next residual in one pass where cycles are launched
+    // one by one (a captured cycle has to end in the buffers it began in) and
+    // no ghost ring has to follow the iterate; a learned start's fallback
+    // changes the iterate between cycles.
+    const bool fused = !use_graphs && !f.px && !f.py && !net;
     // FP64 residual -> FP32 right-hand side, FP32 V-cycle, FP64 update
     return solve_loop(tol, max_cycles, st, [&]() -> int {
         return run_cycle(1, [&]() -> int {
@@ -3392,7 +3551,7 @@ int Multigrid::solve_mixed(double tol, int max_cycles, MgStats *st) {
             KCHECK();
             return 0;
         });
-    });
+    }, fused);
 }
 
 }  // namespace incrmt
