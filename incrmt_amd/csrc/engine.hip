@@ -1792,7 +1792,7 @@ constexpr long long kNoAllocT =
     (long long)((kNoAllocSide + kTileX - 1) / kTileX) * ((kNoAllocSide + kTileY - 1) / kTileY) + 64;
 constexpr size_t a256(long long b) { return (size_t)((b + 255) / 256 * 256); }
 constexpr size_t kNoAllocBytes = 3 * a256(kNoAllocN * 8) + a256(kNoAllocN * 4) + 2 * a256(kNoAllocN) +
-                                 3 * a256(kNoAllocL * 4) + 3 * a256(kNoAllocT * 4) +
+                                 a256(kNoAllocL * 4) + 3 * a256(kNoAllocT * 4) +
                                  a256((kCntIter + kIterSlots) * 4) + a256(16);
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -1886,8 +1886,6 @@ int incrmt_levelset_build_band_noalloc(int m, int n, double ax, double ay, doubl
     w.mark = take(N);
     w.cflag = take(N);
     w.iface = (int *)take(L * 4);
-    w.cand = (int *)take(L * 4);
-    w.pband = (int *)take(L * 4);
     w.tflag = (int *)take(T * 4);
     w.tiles_fim = (int *)take(T * 4);
     w.tiles_ext = (int *)take(T * 4);

@@ -10,7 +10,7 @@
 namespace incrmt {
 
 // Counter slots in LsWork::cnt
-enum { kCntIface = 0, kCntCand, kCntPband, kCntErr, kCntTileFim, kCntTileExt, kCntIter };
+enum { kCntIface = 0, kCntErr, kCntTileFim, kCntTileExt, kCntIter };
 constexpr int kIterSlots = 64;
 enum { kErrNewton = 1, kErrSingular = 2 };
 
@@ -28,7 +28,7 @@ static_assert(kTileThreads % 64 == 0 && kTileThreads <= 1024, "a tile is whole w
 struct LsWork {
     double *va, *vb;      // fixed-point buffers (ghosted grid)
     double *ex, *ey;      // extension values, open marks until they are final (ghosted grid)
-    int *iface, *cand, *pband;  // point lists
+    int *iface;           // interface points
     unsigned char *mark;  // dilation scratch
     unsigned char *cflag; // 1 where a point takes part in the march
     int *tflag;           // per-tile flags: bit 1 march, bit 2 extension

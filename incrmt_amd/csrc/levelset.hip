@@ -27,19 +27,44 @@ namespace {
 
 constexpr int BX = 64, BY = 4;
 
-// Wavefront-aggregated list append: the lanes of a wavefront (among those
-// executing the call) with pred set take consecutive slots of `list` with
-// one atomic on `counter`. The order inside a list carries no meaning: each
-// entry is processed on its own.
-__device__ inline void wave_append(bool pred, int *counter, int *list, int value) {
-    const unsigned long long m = __ballot(pred);
-    if (!m) return;
-    const int lane = __lane_id(), leader = __ffsll((long long)m) - 1;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(counter, __popcll(m));
-    base = __shfl(base, leader, 64);
-    if (pred) list[base + __popcll(m & ((1ull << lane) - 1))] = value;
+// Rows a thread of the scan and of the finalisation takes: a workgroup of
+// BX x BY threads covers BX x (BY kRowSeg) points, whose shared neighbour rows
+// are read once, all loads in flight together.
+constexpr int kRowSeg = 4;
+
+// Workgroup-aggregated list append: bit r of `bits` puts ij0 + r stride on the
+// list, with one atomic on `counter` per workgroup that has any (same-address
+// atomics of a whole launch run one after another: an atomic per wavefront
+// and row made the scan of a circle on 1024^2 take 21.6 us, now 7.5). Every
+// thread of the workgroup calls it. The order inside a list carries no
+// meaning: each entry is processed on its own.
+__device__ inline void block_append(unsigned bits, int ij0, int stride, int *counter, int *list) {
+    __shared__ int tot[BY], base;
+    const int lane = __lane_id(), wave = threadIdx.y;
+    const unsigned long long below = (1ull << lane) - 1;
+    int pos[kRowSeg], n = 0;
+#pragma unroll
+    for (int r = 0; r < kRowSeg; r++) {
+        const unsigned long long m = __ballot(bits >> r & 1);
+        pos[r] = n + __popcll(m & below);
+        n += __popcll(m);
+    }
+    if (lane == 0) tot[wave] = n;
+    __syncthreads();
+    if (lane == 0 && wave == 0) {
+        int all = 0;
+        for (int k = 0; k < BY; k++) all += tot[k];
+        if (all) base = atomicAdd(counter, all);
+    }
+    __syncthreads();
+    if (!n) return;
+    int start = base;
+    for (int k = 0; k < wave; k++) start += tot[k];
+#pragma unroll
+    for (int r = 0; r < kRowSeg; r++)
+        if (bits >> r & 1) list[start + pos[r]] = ij0 + r * stride;
 }
+static_assert(BX == 64, "a row of a workgroup is a wavefront");
 // Wavefront-aggregated flag set: one atomicOr per distinct tile index.
 __device__ inline void wave_flag(bool pred, int *flags, int tile, int bit) {
     unsigned long long m = __ballot(pred);
@@ -53,6 +78,9 @@ __device__ inline void wave_flag(bool pred, int *flags, int tile, int bit) {
     }
 }
 
+inline dim3 grid_rows(const Win &v) {
+    return dim3((v.I1 - v.I0 + BX - 1) / BX, (v.J1 - v.J0 + BY * kRowSeg - 1) / (BY * kRowSeg));
+}
 inline dim3 grid_win(const Win &v) { return dim3((v.I1 - v.I0 + BX - 1) / BX, (v.J1 - v.J0 + BY - 1) / BY); }
 constexpr int kListBlocks = 1024;
 constexpr int kNewtonThreads = 64;  // a wavefront a workgroup: the few there are spread over the chip
@@ -252,7 +280,15 @@ LsGeom geom_of(const Grid &g) {
 }
 
 // ------------------------------------------------------------------ kernels
-__global__ void k_zero_counts(int *cnt, int n) {
+__device__ inline void bbox_clear(int *b) {
+    if (threadIdx.x == 0) {
+        b[0] = b[2] = 1 << 30;
+        b[1] = b[3] = -1;
+    }
+}
+// bbox, when given, starts a rebuild's band box
+__global__ void k_zero_counts(int *cnt, int n, int *bbox = nullptr) {
+    if (bbox) bbox_clear(bbox);
     for (int k = threadIdx.x; k < n; k += blockDim.x) cnt[k] = 0;
 }
 
@@ -277,23 +313,44 @@ __global__ void k_pin(Grid g, ObjConst c, ObjArrays a, Win wn, const double *ix,
 // when a 4-neighbour has the other sign. Interface points are listed for
 // the Newton solves; the fixed-point buffers start at +-inf elsewhere.
 __device__ __forceinline__ void scan_body(const Grid &g, const ObjArrays &a, const LsWork &w, const Win &wn) {
-    const int I = wn.I0 + blockIdx.x * BX + threadIdx.x, J = wn.J0 + blockIdx.y * BY + threadIdx.y;
-    if (I >= wn.I1 || J >= wn.J1) return;
-    const int ij = g.ls(I, J), P = g.P;
-    const double *phi = a.phi;
-    // the four neighbours read together (a neighbour off the grid reads the
-    // point itself, which never differs in sign), then tested
-    const double p0 = phi[ij], pl = phi[I > 0 ? ij - 1 : ij], pr = phi[I < g.ml - 1 ? ij + 1 : ij],
-                 pd = phi[J > 0 ? ij - P : ij], pu = phi[J < g.nl - 1 ? ij + P : ij];
-    const bool pos = p0 > 0;
-    const bool iface = ((pl > 0) != pos) | ((pr > 0) != pos) | ((pd > 0) != pos) | ((pu > 0) != pos);
-    a.st[ij] = pos ? (iface ? 4 : 7) : (iface ? 3 : 0);
-    wave_append(iface, &w.cnt[kCntIface], w.iface, ij);
-    if (!iface) {
-        const double inf = pos ? INFINITY : -INFINITY;
-        w.va[ij] = inf;
-        w.vb[ij] = inf;
+    const int I = wn.I0 + blockIdx.x * BX + threadIdx.x;
+    const int J0 = wn.J0 + (blockIdx.y * BY + threadIdx.y) * kRowSeg, P = g.P;
+    const int ij0 = g.ls(I, J0);
+    unsigned im = 0;  // bit r: row J0 + r is on an interface layer
+    if (I < wn.I1 && J0 < wn.J1) {
+        const double *phi = a.phi;
+        // the points, their neighbours' rows and columns read together (a
+        // neighbour off the grid reads the point nearest to it, which in a row
+        // or column of its own never differs in sign), then tested
+        double pc[kRowSeg + 2], pl[kRowSeg], pr[kRowSeg];
+#pragma unroll
+        for (int r = 0; r < kRowSeg + 2; r++) {
+            const int J = min(max(J0 + r - 1, 0), g.nl - 1);
+            pc[r] = phi[g.ls(I, J)];
+        }
+#pragma unroll
+        for (int r = 0; r < kRowSeg; r++) {
+            const int q = g.ls(I, min(J0 + r, g.nl - 1));
+            pl[r] = phi[I > 0 ? q - 1 : q];
+            pr[r] = phi[I < g.ml - 1 ? q + 1 : q];
+        }
+#pragma unroll
+        for (int r = 0; r < kRowSeg; r++) {
+            if (J0 + r >= wn.J1) break;
+            const int ij = ij0 + r * P;
+            const bool pos = pc[r + 1] > 0;
+            const bool iface = ((pl[r] > 0) != pos) | ((pr[r] > 0) != pos) | ((pc[r] > 0) != pos) |
+                               ((pc[r + 2] > 0) != pos);
+            a.st[ij] = pos ? (iface ? 4 : 7) : (iface ? 3 : 0);
+            if (!iface) {
+                const double inf = pos ? INFINITY : -INFINITY;
+                w.va[ij] = inf;
+                w.vb[ij] = inf;
+            }
+            im |= (unsigned)iface << r;
+        }
     }
+    block_append(im, ij0, P, &w.cnt[kCntIface], w.iface);
 }
 __global__ void k_scan(Grid g, ObjArrays a, LsWork w, Win wn) { scan_body(g, a, w, wn); }
 
@@ -325,27 +382,46 @@ __global__ __launch_bounds__(kNewtonThreads) void k_newton(Grid g, LsGeom lg, Ob
 // Candidate points: non-interface points within R cells (max norm) of an
 // interface point, R covering the band cut-offs; separable dilation, rows
 // then columns.
+// A wavefront is 64 columns of a row: the interface flags of its columns and of
+// the 64 on either side (more for R > 64) are three votes, and a point's window is
+// a range of their bits, instead of 2R + 1 reads a point (5.7 -> 4.2 us for a
+// circle on 1024^2, 26.7 -> 13.0 us for 2048^2 whole).
 __device__ __forceinline__ void dilate_rows_body(const Grid &g, const ObjArrays &a, const LsWork &w, int R,
                                                  const Win &wn) {
-    const int I = wn.I0 + blockIdx.x * BX + threadIdx.x, J = wn.J0 + blockIdx.y * BY + threadIdx.y;
-    if (I >= wn.I1 || J >= wn.J1) return;
-    const int ij = g.ls(I, J);
-    // every read of the range issued without waiting on the one before (the
-    // OR over it is the same with or without stopping at the first hit)
-    const int d0 = I - R < 0 ? -I : -R, d1 = I + R >= g.ml ? g.ml - 1 - I : R;
-    bool hit = false;
-#pragma unroll 4
-    for (int d = d0; d <= d1; d++) {
-        const int s = a.st[ij + d];
-        hit |= s == 3 || s == 4;
+    const int I = wn.I0 + blockIdx.x * BX + threadIdx.x, lane = threadIdx.x;
+    const int J0 = wn.J0 + (blockIdx.y * BY + threadIdx.y) * kRowSeg;
+    const int far = (R + 63) / 64;
+    unsigned hit = 0;
+    for (int k = -far; k <= far; k++) {
+        const int Ik = I + 64 * k;
+        const bool in = Ik >= 0 && Ik < g.ml;
+        int st[kRowSeg];
+#pragma unroll
+        for (int r = 0; r < kRowSeg; r++) {
+            const int s = a.st[g.ls(min(max(Ik, 0), g.ml - 1), min(J0 + r, g.nl - 1))];
+            st[r] = in ? s : 0;
+        }
+        // the bits of this group within R of the lane's point
+        const int lo = max(lane - R - 64 * k, 0), hi = min(lane + R - 64 * k, 63);
+        const unsigned long long win = lo > hi ? 0 : (~0ull >> (63 - hi)) & (~0ull << lo);
+#pragma unroll
+        for (int r = 0; r < kRowSeg; r++) {
+            const unsigned long long m = __ballot(st[r] == 3 || st[r] == 4);
+            hit |= (unsigned)((m & win) != 0) << r;
+        }
     }
-    w.mark[ij] = hit;
+    if (I >= wn.I1) return;
+#pragma unroll
+    for (int r = 0; r < kRowSeg; r++)
+        if (J0 + r < wn.J1) w.mark[g.ls(I, J0 + r)] = hit >> r & 1;
 }
 __global__ void k_dilate_rows(Grid g, ObjArrays a, LsWork w, int R, Win wn) { dilate_rows_body(g, a, w, R, wn); }
 // The column pass: a thread takes kColSeg consecutive rows of one column and
 // keeps the count of marked points in the column window [J - R, J + R]
 // (clipped to the grid) as it slides down, one point in and one out per row,
-// instead of reading the 2R + 1 marks of every point.
+// instead of reading the 2R + 1 marks of every point. Bound by latency: the
+// reads of the first window go out eight at a time, the sliding ones with them
+// (13.1 -> 5.4 us for a circle on 1024^2).
 constexpr int kColSeg = 8;
 static_assert(kTileY >= kColSeg, "a thread's rows span at most two tile rows");
 inline dim3 grid_win_cols(const Win &v) {
@@ -358,45 +434,41 @@ __device__ __forceinline__ void dilate_cols_body(const Grid &g, const ObjArrays 
     const bool col = I < wn.I1 && J0 < wn.J1;
     const unsigned char *mk = w.mark + (col ? g.ls(I, 0) : 0);
     int cnt = 0;
-    if (col) {
-        const int lo = J0 - R < 0 ? 0 : J0 - R, hi = J0 + R >= g.nl ? g.nl - 1 : J0 + R;
-#pragma unroll 4
-        for (int J = lo; J <= hi; J++) cnt += mk[J * g.P] != 0;
-    }
     unsigned hm = 0;  // bit k: row J0 + k is a candidate
+    if (col) {
+        // the points' statuses and the marks entering and leaving the sliding
+        // window are read ahead of the first window's count
+        int st[kColSeg], in[kColSeg], out[kColSeg];
 #pragma unroll
-    for (int k = 0; k < kColSeg; k++) {
-        const int J = J0 + k;
-        const bool in = col && J < wn.J1;
-        if (in && k > 0) {
-            // the window moves from [J-1-R, J-1+R] to [J-R, J+R]
-            if (J + R < g.nl) cnt += mk[(J + R) * g.P] != 0;
-            if (J - 1 - R >= 0) cnt -= mk[(J - 1 - R) * g.P] != 0;
+        for (int k = 0; k < kColSeg; k++) {
+            const int J = min(J0 + k, g.nl - 1);
+            st[k] = a.st[g.ls(I, J)];
+            const int a1 = J0 + k + R, a0 = J0 + k - 1 - R;
+            const int m1 = mk[min(a1, g.nl - 1) * g.P], m0 = mk[max(a0, 0) * g.P];
+            in[k] = k > 0 && a1 < g.nl && m1 != 0;
+            out[k] = k > 0 && a0 >= 0 && m0 != 0;
         }
-        if (in) {
-            const int ij = g.ls(I, J), s = a.st[ij];
-            const bool hit = s != 3 && s != 4 && cnt > 0;
-            w.cflag[ij] = hit;
+        const int lo = J0 - R < 0 ? 0 : J0 - R, hi = J0 + R >= g.nl ? g.nl - 1 : J0 + R;
+        for (int J = lo; J <= hi; J += 8) {
+            int m[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) m[k] = mk[min(J + k, hi) * g.P];
+#pragma unroll
+            for (int k = 0; k < 8; k++) cnt += J + k <= hi && m[k] != 0;
+        }
+#pragma unroll
+        for (int k = 0; k < kColSeg; k++) {
+            const int J = J0 + k;
+            if (J >= wn.J1) break;
+            // the window moves from [J-1-R, J-1+R] to [J-R, J+R]
+            cnt += in[k] - out[k];
+            const bool hit = st[k] != 3 && st[k] != 4 && cnt > 0;
+            w.cflag[g.ls(I, J)] = hit;
             hm |= (unsigned)hit << k;
         }
     }
-    // the candidates of the whole wavefront appended with one atomic (an
-    // inclusive prefix count across the lanes), and the tile flags set once
-    // per wavefront and tile row: a thread's rows span at most two tile rows
-    const int lane = __lane_id(), nh = __popc(hm);
-    int incl = nh;
-    for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += v;
-    }
-    const int total = __shfl(incl, 63, 64);
-    int base = 0;
-    if (lane == 63 && total > 0) base = atomicAdd(&w.cnt[kCntCand], total);
-    base = __shfl(base, 63, 64);
-    int pos = base + incl - nh;
-#pragma unroll
-    for (int k = 0; k < kColSeg; k++)
-        if ((hm >> k) & 1) w.cand[pos++] = g.ls(I, J0 + k);
+    // the tile flags set once per wavefront and tile row: a thread's rows span
+    // at most two tile rows
     const int ta = J0 / kTileY, tb = (J0 + kColSeg - 1) / kTileY;
     unsigned ma = 0;  // rows of tile row ta
 #pragma unroll
@@ -406,13 +478,6 @@ __device__ __forceinline__ void dilate_cols_body(const Grid &g, const ObjArrays 
     if (tb != ta) wave_flag((hm & ~ma) != 0, w.tflag, tb * w.ntx + I / kTileX, 1);
 }
 __global__ void k_dilate_cols(Grid g, ObjArrays a, LsWork w, int R, Win wn) { dilate_cols_body(g, a, w, R, wn); }
-
-__global__ void k_bbox_init(LsWork w) {
-    if (threadIdx.x == 0) {
-        w.bbox[0] = w.bbox[2] = 1 << 30;
-        w.bbox[1] = w.bbox[3] = -1;
-    }
-}
 
 // Collect the tiles whose flag has `bit` set into a list, clearing the bit.
 __device__ __forceinline__ void compact_tiles_body(const LsWork &w, int bit, int *list, int slot) {
@@ -600,82 +665,115 @@ __global__ __launch_bounds__(kTileThreads) void k_fim_tiles_batch(Grid g, EikGeo
 // fixed-point values and status 5/2, points the heap would have left in its
 // queue status 6/1, everything outside the band the cut-off value. Outside
 // band points are listed for the extension.
-__device__ void finalize_point(Grid g, ObjConst c, ObjArrays a, LsWork w, const double *v, int I, int J,
-                               int (*bb)[BX * BY], int lane);
+// Bound by latency: a thread's four points share their neighbours' rows, every
+// load is issued before the first test (29.6 -> 12.7 us for a circle
+// on 1024^2), the band's box is formed from votes, and an atomic goes out only
+// where it widens the box that the launch has so far.
 __device__ __forceinline__ void finalize_body(const Grid &g, const ObjConst &c, const ObjArrays &a, const LsWork &w,
                                               const double *v, const Win &wn) {
-    __shared__ int bb[4][BX * BY];
-    const int t = threadIdx.y * BX + threadIdx.x;
-    bb[0][t] = bb[2][t] = 1 << 30;
-    bb[1][t] = bb[3][t] = -1;
-    const int I = wn.I0 + blockIdx.x * BX + threadIdx.x, J = wn.J0 + blockIdx.y * BY + threadIdx.y;
-    if (I < wn.I1 && J < wn.J1) finalize_point(g, c, a, w, v, I, J, bb, t);
+    __shared__ int box[4];
+    const int t = threadIdx.y * BX + threadIdx.x, lane = threadIdx.x;
+    if (t < 4) box[t] = t & 1 ? -1 : 1 << 30;
+    const int I = wn.I0 + blockIdx.x * BX + threadIdx.x;
+    const int J0 = wn.J0 + (blockIdx.y * BY + threadIdx.y) * kRowSeg;
+    const double lim = c.phi_up, dlim = c.phi_down;
+    unsigned nm = 0, pm = 0;  // bit r: row J0 + r in the band or its trial points; outside band
+    if (I < wn.I1 && J0 < wn.J1) {
+        // a point outside the band tests its four neighbours (one off the grid
+        // counts as not accepted)
+        int sc[kRowSeg + 2], sl[kRowSeg], sr[kRowSeg];
+        double vc[kRowSeg + 2], vl[kRowSeg], vr[kRowSeg];
+        const bool hl = I > 0, hr = I < g.ml - 1;
+#pragma unroll
+        for (int r = 0; r < kRowSeg + 2; r++) {
+            const int q = g.ls(I, min(max(J0 + r - 1, 0), g.nl - 1));
+            sc[r] = a.st[q];
+            vc[r] = v[q];
+        }
+#pragma unroll
+        for (int r = 0; r < kRowSeg; r++) {
+            const int q = g.ls(I, min(J0 + r, g.nl - 1)), ql = hl ? q - 1 : q, qr = hr ? q + 1 : q;
+            sl[r] = a.st[ql];
+            vl[r] = v[ql];
+            sr[r] = a.st[qr];
+            vr[r] = v[qr];
+        }
+        auto acc_pos = [&](int s, double x) { return s == 4 || (s == 7 && x < lim); };
+        auto acc_neg = [&](int s, double x) { return s == 3 || (s == 0 && x > dlim); };
+#pragma unroll
+        for (int r = 0; r < kRowSeg; r++) {
+            const int J = J0 + r;
+            if (J >= wn.J1) break;
+            const bool hd = J > 0, hu = J < g.nl - 1;
+            auto any_nb = [&](auto acc) {
+                return (hl && acc(sl[r], vl[r])) | (hr && acc(sr[r], vr[r])) | (hd && acc(sc[r], vc[r])) |
+                       (hu && acc(sc[r + 2], vc[r + 2]));
+            };
+            const int s = sc[r + 1], ij = g.ls(I, J);
+            const double v0 = vc[r + 1];
+            int ns = s;
+            double phi;
+            if (s == 3 || s == 4) {
+                phi = v0;
+            } else if (s == 7) {
+                if (v0 < lim) { ns = 5; phi = v0; }
+                else {
+                    ns = any_nb(acc_pos) ? 6 : 7;
+                    phi = lim;
+                }
+            } else {
+                if (v0 > dlim) { ns = 2; phi = v0; }
+                else {
+                    ns = any_nb(acc_neg) ? 1 : 0;
+                    phi = dlim;
+                }
+            }
+            w.mark[ij] = (unsigned char)ns;  // statuses go to st after every thread read the old ones
+            a.phi[ij] = phi;
+            nm |= (unsigned)(ns >= 1 && ns <= 6) << r;
+            pm |= (unsigned)(ns == 4 || ns == 5) << r;
+        }
+    }
+    // outside band points mark their tile for the extension
+    const int ta = J0 / kTileY, tb = (J0 + kRowSeg - 1) / kTileY;
+    unsigned ma = 0;  // rows of tile row ta
+#pragma unroll
+    for (int r = 0; r < kRowSeg; r++)
+        if ((J0 + r) / kTileY == ta) ma |= 1u << r;
+    wave_flag((pm & ma) != 0, w.tflag, ta * w.ntx + I / kTileX, 2);
+    if (tb != ta) wave_flag((pm & ~ma) != 0, w.tflag, tb * w.ntx + I / kTileX, 2);
     // bounding box of the band and its trial points, for the next window
     __syncthreads();
-    for (int h = BX * BY / 2; h > 0; h >>= 1) {
-        if (t < h) {
-            bb[0][t] = min(bb[0][t], bb[0][t + h]);
-            bb[1][t] = max(bb[1][t], bb[1][t + h]);
-            bb[2][t] = min(bb[2][t], bb[2][t + h]);
-            bb[3][t] = max(bb[3][t], bb[3][t + h]);
+    const unsigned long long cols = __ballot(nm != 0);
+    if (cols) {
+        int lo = kRowSeg, hi = 0;
+#pragma unroll
+        for (int r = 0; r < kRowSeg; r++)
+            if (__ballot(nm >> r & 1)) { lo = min(lo, r); hi = r; }
+        if (lane == 0) {
+            atomicMin(&box[0], I + __ffsll((long long)cols) - 1);
+            atomicMax(&box[1], I + 63 - __clzll((long long)cols));
+            atomicMin(&box[2], J0 + lo);
+            atomicMax(&box[3], J0 + hi);
         }
-        __syncthreads();
     }
-    if (t == 0 && bb[1][0] >= 0) {
-        atomicMin(&w.bbox[0], bb[0][0]);
-        atomicMax(&w.bbox[1], bb[1][0]);
-        atomicMin(&w.bbox[2], bb[2][0]);
-        atomicMax(&w.bbox[3], bb[3][0]);
+    __syncthreads();
+    if (t < 4 && box[1] >= 0) {
+        const int b = box[t], now = __hip_atomic_load(&w.bbox[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (t & 1) { if (b > now) atomicMax(&w.bbox[t], b); }
+        else if (b < now) atomicMin(&w.bbox[t], b);
     }
 }
 __global__ void k_finalize(Grid g, ObjConst c, ObjArrays a, LsWork w, const double *v, Win wn) {
     finalize_body(g, c, a, w, v, wn);
 }
-__device__ void finalize_point(Grid g, ObjConst c, ObjArrays a, LsWork w, const double *v, int I, int J,
-                               int (*bb)[BX * BY], int lane) {
-    const int ij = g.ls(I, J), P = g.P, s = a.st[ij];
-    const double lim = c.phi_up, dlim = c.phi_down;
-    // a point outside the band tests its four neighbours: their statuses
-    // and values are read together (a neighbour off the grid reads the point
-    // itself and is masked out)
-    const bool hl = I > 0, hr = I < g.ml - 1, hd = J > 0, hu = J < g.nl - 1;
-    const int ql = hl ? ij - 1 : ij, qr = hr ? ij + 1 : ij, qd = hd ? ij - P : ij, qu = hu ? ij + P : ij;
-    auto any_nb = [&](auto acc) {
-        const int tl = a.st[ql], tr = a.st[qr], td = a.st[qd], tu = a.st[qu];
-        const double vl = v[ql], vr = v[qr], vd = v[qd], vu = v[qu];
-        return (hl && acc(tl, vl)) | (hr && acc(tr, vr)) | (hd && acc(td, vd)) | (hu && acc(tu, vu));
-    };
-    auto acc_pos = [&](int t, double x) { return t == 4 || (t == 7 && x < lim); };
-    auto acc_neg = [&](int t, double x) { return t == 3 || (t == 0 && x > dlim); };
-    const double v0 = v[ij];
-    int ns = s;
-    double phi;
-    if (s == 3 || s == 4) {
-        phi = v0;
-    } else if (s == 7) {
-        if (v0 < lim) { ns = 5; phi = v0; }
-        else {
-            ns = any_nb(acc_pos) ? 6 : 7;
-            phi = lim;
-        }
-    } else {
-        if (v0 > dlim) { ns = 2; phi = v0; }
-        else {
-            ns = any_nb(acc_neg) ? 1 : 0;
-            phi = dlim;
-        }
-    }
-    w.mark[ij] = (unsigned char)ns;  // statuses go to st after every thread read the old ones
-    if (ns >= 1 && ns <= 6) {
-        bb[0][lane] = I; bb[1][lane] = I; bb[2][lane] = J; bb[3][lane] = J;
-    }
-    a.phi[ij] = phi;
-    const bool pb = ns == 4 || ns == 5;
-    wave_append(pb, &w.cnt[kCntPband], w.pband, ij);
-    wave_flag(pb, w.tflag, (J / kTileY) * w.ntx + I / kTileX, 2);
-}
+// The new statuses, and the band's box to the host (work sets that keep a
+// window): a copy command behind the kernels cost as much as a launch, one per
+// solid.
 __device__ __forceinline__ void commit_status_body(const Grid &g, const ObjArrays &a, const LsWork &w, const Win &wn) {
     const int I = wn.I0 + blockIdx.x * BX + threadIdx.x, J = wn.J0 + blockIdx.y * BY + threadIdx.y;
+    if (w.hbbox && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.y == 0 && threadIdx.x < 4)
+        w.hbbox[threadIdx.x] = w.bbox[threadIdx.x];
     if (I >= wn.I1 || J >= wn.J1) return;
     const int ij = g.ls(I, J);
     a.st[ij] = w.mark[ij];
@@ -1199,8 +1297,10 @@ __global__ void k_pin_b(Grid g, const SetupItem *it) {
     const SetupItem &x = it[blockIdx.z];
     if (x.pin) pin_body(g, x.c, x.a, x.wn, x.pin_x, x.pin_y);
 }
-__global__ void k_counts_b(const SetupItem *it, int from, int n) {
-    int *cnt = it[blockIdx.z].w.cnt + from;
+// starts a rebuild's counters and band box
+__global__ void k_counts_b(const SetupItem *it, int n) {
+    int *cnt = it[blockIdx.z].w.cnt;
+    bbox_clear(it[blockIdx.z].w.bbox);
     for (int k = threadIdx.x; k < n; k += blockDim.x) cnt[k] = 0;
 }
 __global__ void k_scan_b(Grid g, const SetupItem *it) {
@@ -1224,14 +1324,6 @@ __global__ void k_compact_tiles_b(const SetupItem *it, int ext) {
     if (ext) compact_tiles_body(w, 2, w.tiles_ext, kCntTileExt);
     else compact_tiles_body(w, 1, w.tiles_fim, kCntTileFim);
 }
-__global__ void k_bbox_init_b(const SetupItem *it) {
-    const LsWork &w = it[blockIdx.z].w;
-    if (threadIdx.x == 0) {
-        w.cnt[kCntPband] = 0;
-        w.bbox[0] = w.bbox[2] = 1 << 30;
-        w.bbox[1] = w.bbox[3] = -1;
-    }
-}
 __global__ void k_finalize_b(Grid g, const SetupItem *it) {
     const SetupItem &x = it[blockIdx.z];
     finalize_body(g, x.c, x.a, x.w, x.v, x.wn);
@@ -1253,13 +1345,17 @@ __global__ void k_commit_status_b(Grid g, const SetupItem *it) {
 // max_passes pass without convergence, or a HIP error.
 // Its two halves: enqueue one batch of passes (starting at pass `passes`)
 // with the read-back of its counters, and, once the stream has run them,
-// decide from the counters whether the iteration has ended.
+// decide from the counters whether the iteration has ended. zeroed: the
+// first batch's counters are zero already (a rebuild's set-up cleared them).
 template <class F>
-int iter_enqueue(hipStream_t s, LsWork &w, int predict, int passes, F pass, int &batch, int least = 2) {
+int iter_enqueue(hipStream_t s, LsWork &w, int predict, int passes, F pass, int &batch, int least = 2,
+                 bool zeroed = false) {
     batch = predict < least ? least : predict;
     if (batch > kIterSlots) batch = kIterSlots;
-    k_zero_counts<<<1, 64, 0, s>>>(w.cnt + kCntIter, kIterSlots);
-    KCHECK();
+    if (passes || !zeroed) {
+        k_zero_counts<<<1, 64, 0, s>>>(w.cnt + kCntIter, kIterSlots);
+        KCHECK();
+    }
     for (int b = 0; b < batch; b++)
         if (int rc = pass(passes + b, b)) return rc;
     HIP_CHECK(hipMemcpyAsync(w.hcnt, w.cnt, (kCntIter + kIterSlots) * sizeof(int), hipMemcpyDeviceToHost, s));
@@ -1281,11 +1377,12 @@ bool iter_done(LsWork &w, int &predict, int &passes, int batch, int *passes_out)
     return false;
 }
 template <class F>
-int iterate(hipStream_t s, LsWork &w, int &predict, int max_passes, F pass, int *passes_out, int least = 2) {
+int iterate(hipStream_t s, LsWork &w, int &predict, int max_passes, F pass, int *passes_out, int least = 2,
+            bool zeroed = false) {
     int passes = 0;
     while (passes < max_passes) {
         int batch;
-        if (int rc = iter_enqueue(s, w, predict, passes, pass, batch, least)) return rc;
+        if (int rc = iter_enqueue(s, w, predict, passes, pass, batch, least, zeroed)) return rc;
         HIP_CHECK(hipStreamSynchronize(s));
         if (iter_done(w, predict, passes, batch, passes_out)) return 0;
     }
@@ -1429,8 +1526,6 @@ int ls_alloc(const Grid &g, LsWork &w, hipStream_t s) {
     }
     const size_t L = (size_t)g.ml * g.nl + 64;
     HIP_CHECK(hipMalloc((void **)&w.iface, L * sizeof(int)));
-    HIP_CHECK(hipMalloc((void **)&w.cand, L * sizeof(int)));
-    HIP_CHECK(hipMalloc((void **)&w.pband, L * sizeof(int)));
     HIP_CHECK(hipMalloc((void **)&w.mark, N));
     HIP_CHECK(memset_sync(w.mark, 0, N, s));
     HIP_CHECK(hipMalloc((void **)&w.cflag, N));
@@ -1451,7 +1546,7 @@ int ls_alloc(const Grid &g, LsWork &w, hipStream_t s) {
 }
 
 void ls_free(LsWork &w) {
-    void *p[] = {w.va, w.vb, w.ex, w.ey, w.iface, w.cand, w.pband, w.mark, w.cflag, w.tflag,
+    void *p[] = {w.va, w.vb, w.ex, w.ey, w.iface, w.mark, w.cflag, w.tflag,
                  w.tiles_fim, w.tiles_ext, w.cnt, w.bbox};
     for (auto q : p)
         if (q) (void)hipFree(q);
@@ -1520,13 +1615,13 @@ static int rebuild_setup(hipStream_t s, const Grid &g, const ObjConst &c, const 
         k_pin<<<grid_win(wn), bb, 0, s>>>(g, c, a, wn, pin_x, pin_y);
         KCHECK();
     }
-    k_zero_counts<<<1, 64, 0, s>>>(w.cnt, kCntIter + kIterSlots);
+    k_zero_counts<<<1, 64, 0, s>>>(w.cnt, kCntIter + kIterSlots, w.bbox);
     KCHECK();
-    k_scan<<<grid_win(wn), bb, 0, s>>>(g, a, w, wn);
+    k_scan<<<grid_rows(wn), bb, 0, s>>>(g, a, w, wn);
     KCHECK();
     k_newton<<<kListBlocks, kNewtonThreads, 0, s>>>(g, geom_of(g), a, w);
     KCHECK();
-    k_dilate_rows<<<grid_win(wr), bb, 0, s>>>(g, a, w, R < g.ml ? R : g.ml, wr);
+    k_dilate_rows<<<grid_rows(wr), bb, 0, s>>>(g, a, w, R < g.ml ? R : g.ml, wr);
     KCHECK();
     k_dilate_cols<<<grid_win_cols(wn), bb, 0, s>>>(g, a, w, R < g.nl ? R : g.nl, wn);
     KCHECK();
@@ -1535,11 +1630,10 @@ static int rebuild_setup(hipStream_t s, const Grid &g, const ObjConst &c, const 
     return 0;
 }
 
-// The host side of a rebuild's finish (after the finalisation): the band
-// box's read-back and the window the next rebuild grows from.
+// The host side of a rebuild's finish (after its last kernel, which writes the
+// band's box to the host): the event to wait for and the window the next rebuild grows from.
 static int finish_window(hipStream_t s, LsWork &w, const Win &wn, bool whole) {
     if (w.ev_bbox) {  // a work set without the event keeps no window (one-off rebuilds)
-        HIP_CHECK(hipMemcpyAsync(w.hbbox, w.bbox, 4 * sizeof(int), hipMemcpyDeviceToHost, s));
         HIP_CHECK(hipEventRecord(w.ev_bbox, s));
         w.bbox_pending = true;
     }
@@ -1556,18 +1650,13 @@ static int rebuild_finish(hipStream_t s, const Grid &g, const ObjConst &c, const
                           const Win &wn, bool whole, int passes) {
     const dim3 bb(BX, BY);
     double *bufs[2] = {w.va, w.vb};
-    k_zero_counts<<<1, 64, 0, s>>>(w.cnt + kCntPband, 1);
+    k_finalize<<<grid_rows(wn), bb, 0, s>>>(g, c, a, w, bufs[passes & 1], wn);
     KCHECK();
-    k_bbox_init<<<1, 64, 0, s>>>(w);
-    KCHECK();
-    k_finalize<<<grid_win(wn), bb, 0, s>>>(g, c, a, w, bufs[passes & 1], wn);
-    KCHECK();
-    if (int rc = finish_window(s, w, wn, whole)) return rc;
     k_compact_tiles<<<64, 256, 0, s>>>(w, 2, w.tiles_ext, kCntTileExt);
     KCHECK();
     k_commit_status<<<grid_win(wn), bb, 0, s>>>(g, a, w, wn);
     KCHECK();
-    return 0;
+    return finish_window(s, w, wn, whole);
 }
 
 constexpr int kMaxFimPasses = 4096;
@@ -1591,7 +1680,7 @@ static int rebuild_common(hipStream_t s, const Grid &g, const ObjConst &c, const
     eg.init(g.dx, g.dy);
     int passes = 0;
     int rc = iterate(s, w, w.pred_fim, kMaxFimPasses,
-                     [&](int p, int slot) { return fim_pass(s, g, eg, c, a, w, p, slot); }, &passes);
+                     [&](int p, int slot) { return fim_pass(s, g, eg, c, a, w, p, slot); }, &passes, 2, true);
     if (rc) return rc;
     if (w.hcnt[kCntErr] & kErrNewton) return 3;
     if (fim_iters) *fim_iters = passes;
@@ -1627,10 +1716,11 @@ static const SetupItem *upload_items(hipStream_t s, LsBatch &bt, int region, con
     return d;
 }
 // a grid covering the largest of the items' windows (rows: their row windows)
-static dim3 grid_items(const std::vector<SetupItem> &v, bool rows, bool cols = false) {
+template <class F>
+static dim3 grid_items(const std::vector<SetupItem> &v, F grid) {
     unsigned gx = 1, gy = 1;
     for (const SetupItem &x : v) {
-        const dim3 d = cols ? grid_win_cols(x.wn) : grid_win(rows ? x.wr : x.wn);
+        const dim3 d = grid(x);
         gx = std::max(gx, d.x);
         gy = std::max(gy, d.y);
     }
@@ -1684,14 +1774,16 @@ int ls_pin_rebuild_batch_begin(hipStream_t s, const Grid &g, const std::vector<L
     int rc = 0;
     const SetupItem *d = upload_items(s, bt, 0, p->su, &rc);
     if (rc) return rc;
-    const dim3 bb(BX, BY), gw = grid_items(p->su, false), gr = grid_items(p->su, true),
-               gc = grid_items(p->su, false, true);
+    const dim3 bb(BX, BY), gw = grid_items(p->su, [](const SetupItem &x) { return grid_win(x.wn); }),
+               gs = grid_items(p->su, [](const SetupItem &x) { return grid_rows(x.wn); }),
+               gr = grid_items(p->su, [](const SetupItem &x) { return grid_rows(x.wr); }),
+               gc = grid_items(p->su, [](const SetupItem &x) { return grid_win_cols(x.wn); });
     const unsigned m = (unsigned)p->su.size();
     k_pin_b<<<gw, bb, 0, s>>>(g, d);
     KCHECK();
-    k_counts_b<<<dim3(1, 1, m), 64, 0, s>>>(d, 0, kCntIter + kIterSlots);
+    k_counts_b<<<dim3(1, 1, m), 64, 0, s>>>(d, kCntIter + kIterSlots);
     KCHECK();
-    k_scan_b<<<gw, bb, 0, s>>>(g, d);
+    k_scan_b<<<gs, bb, 0, s>>>(g, d);
     KCHECK();
     k_newton_b<<<dim3(list_blocks(m), 1, m), kNewtonThreads, 0, s>>>(g, geom_of(g), d);
     KCHECK();
@@ -1738,18 +1830,17 @@ int ls_pin_rebuild_batch_end(hipStream_t s, const Grid &g, const std::vector<LsJ
         int e = 0;
         const SetupItem *d = upload_items(s, bt, 1, p->su, &e);
         if (e) return e;
-        const dim3 bb(BX, BY), gw = grid_items(p->su, false);
+        const dim3 bb(BX, BY), gw = grid_items(p->su, [](const SetupItem &x) { return grid_win(x.wn); }),
+                   gs = grid_items(p->su, [](const SetupItem &x) { return grid_rows(x.wn); });
         const unsigned m = (unsigned)p->su.size();
-        k_bbox_init_b<<<dim3(1, 1, m), 64, 0, s>>>(d);
+        k_finalize_b<<<gs, bb, 0, s>>>(g, d);
         KCHECK();
-        k_finalize_b<<<gw, bb, 0, s>>>(g, d);
-        KCHECK();
-        for (size_t t = 0; t < p->who.size(); t++)
-            if ((e = finish_window(s, *jobs[p->who[t]].w, p->wn[p->who[t]], p->whole[p->who[t]]))) return e;
         k_compact_tiles_b<<<dim3(64, 1, m), 256, 0, s>>>(d, 1);
         KCHECK();
         k_commit_status_b<<<gw, bb, 0, s>>>(g, d);
         KCHECK();
+        for (size_t t = 0; t < p->who.size(); t++)
+            if ((e = finish_window(s, *jobs[p->who[t]].w, p->wn[p->who[t]], p->whole[p->who[t]]))) return e;
         if (fim_iters) *fim_iters = most;
         return 0;
     }();
@@ -1788,7 +1879,7 @@ int ls_pin_rebuild_begin(hipStream_t s, const Grid &g, const ObjConst &c, const 
     if (!r.live) return 0;
     r.eg.init(g.dx, g.dy);
     return iter_enqueue(s, w, w.pred_fim, 0,
-                        [&](int p, int slot) { return fim_pass(s, g, r.eg, c, a, w, p, slot); }, r.batch);
+                        [&](int p, int slot) { return fim_pass(s, g, r.eg, c, a, w, p, slot); }, r.batch, 2, true);
 }
 
 int ls_pin_rebuild_end(hipStream_t s, const Grid &g, const ObjConst &c, const ObjArrays &a, LsWork &w, LsRebuild &r,
