@@ -1554,12 +1554,81 @@ __global__ void k_apply(int kind, LevelArgs a, FemC k, const double *x, const do
 }
 
 // ------------------------------------------------------------- reductions
-// Partial sums per block of (b^2, r^2, b) over level 0 with r = b - A z.
+// The end of a reduction over level 0 within the kernel that forms it: each
+// workgroup's sums of three values, then, in the workgroup that comes last, the
+// sum of all in the fixed order of k_sum_partials (a launch of its own for it
+// took 3.8 us and a gap, eight times a step; in the kernel it takes 1.5 us up to
+// 256^2 points and 5 us with all workgroups: a step at 64^2 1.15 -> 1.13 ms, at
+// 1024^2 the same). host: pinned memory for the result, or null.
+// The partial sums go out past the XCDs' caches and are waited for before the
+// workgroup takes its ticket, so the last one's reads, which pass the caches too,
+// find them all; a release fence would write back every line that the kernel
+// has dirtied. Tickets in groups of 32: additions to one address run one after
+// another. The last workgroup clears them for the next launch.
+// red: [0] to [2] the result, then the partial sums and the tickets.
+constexpr int kRedGroup = 32, kRedTickets = 1 + kRedBlocks / kRedGroup;
+constexpr size_t red_bytes() { return (8 + 3 * kRedBlocks) * sizeof(double) + kRedTickets * sizeof(int); }
+// Workgroups of a reduction over n points, which p0 and the stride kRedStride walk:
+// those beyond the points would add zeros.
+constexpr int kRedStride = kRedBlocks * kRedThreads;
+inline int red_blocks(long long n) {
+    const long long b = (n + kRedThreads - 1) / kRedThreads;
+    return b < kRedBlocks ? (int)b : kRedBlocks;
+}
+// The sum of v over the workgroup, in thread 0, as the tree over halves adds it.
+__device__ void block_tree3(double (&v)[3]) {
+    static_assert(kRedThreads == 256, "two halvings through LDS, the rest within a wavefront");
+    __shared__ double s[3][128];
+    const int t = threadIdx.x;
+    for (int h = 128; h >= 64; h /= 2) {
+        if (t >= h && t < 2 * h)
+            for (int k = 0; k < 3; k++) s[k][t - h] = v[k];
+        __syncthreads();
+        if (t < h)
+            for (int k = 0; k < 3; k++) v[k] += s[k][t];
+        __syncthreads();
+    }
+    if (t < 64)
+        for (int h = 32; h > 0; h /= 2)
+            for (int k = 0; k < 3; k++) v[k] += __shfl_down(v[k], h, 64);
+}
+__device__ void reduce_all(double (&v)[3], double *red, double *host) {
+    __shared__ int last;
+    double *part = red + 8;
+    int *tickets = (int *)(part + 3 * kRedBlocks);
+    const int t = threadIdx.x, b = blockIdx.x, nb = gridDim.x;
+    block_tree3(v);
+    if (t == 0) {
+        for (int k = 0; k < 3; k++)
+            __hip_atomic_store(&part[3 * b + k], v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        asm volatile("" ::: "memory");
+        const int grp = b / kRedGroup, ngrp = (nb + kRedGroup - 1) / kRedGroup;
+        const int members = grp + 1 < ngrp ? kRedGroup : nb - grp * kRedGroup;
+        last = 0;
+        if (__hip_atomic_fetch_add(&tickets[1 + grp], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == members - 1)
+            last = __hip_atomic_fetch_add(&tickets[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == ngrp - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    double w[3] = {0, 0, 0};
+    for (int p = t; p < nb; p += kRedThreads)
+        for (int k = 0; k < 3; k++)
+            w[k] += __hip_atomic_load(&part[3 * p + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t < kRedTickets) __hip_atomic_store(&tickets[t], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    block_tree3(w);
+    if (t == 0)
+        for (int k = 0; k < 3; k++) {
+            red[k] = w[k];
+            if (host) host[k] = w[k];  // no copy behind the kernel
+        }
+}
+// The sums of b^2, r^2 and b over level 0 with r = b - A z.
 __global__ void k_norms(int kind, LevelArgs a, FemC k, const double *z, const double *b, const double *fw,
-                        const double *fs, const double *kc, double *part) {
-    __shared__ double s0[kRedThreads], s1[kRedThreads], s2[kRedThreads];
+                        const double *fs, const double *kc, double *red, double *host) {
     double bb = 0, rr = 0, bs = 0;
-    const int N = a.nx * a.ny, S = gridDim.x * blockDim.x, di = S % a.nx, dj = S / a.nx;
+    const int N = a.nx * a.ny, S = kRedStride, di = S % a.nx, dj = S / a.nx;
     // point p = j nx + i, stepped by S without a division per point; the
     // unrolled iterations' loads are in flight together (the sums keep
     // their order)
@@ -1577,22 +1646,11 @@ __global__ void k_norms(int kind, LevelArgs a, FemC k, const double *z, const do
         j += dj;
         if (i >= a.nx) { i -= a.nx; j++; }
     }
-    s0[threadIdx.x] = bb; s1[threadIdx.x] = rr; s2[threadIdx.x] = bs;
-    __syncthreads();
-    for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-            s0[threadIdx.x] += s0[threadIdx.x + w];
-            s1[threadIdx.x] += s1[threadIdx.x + w];
-            s2[threadIdx.x] += s2[threadIdx.x + w];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        part[3 * blockIdx.x] = s0[0]; part[3 * blockIdx.x + 1] = s1[0]; part[3 * blockIdx.x + 2] = s2[0];
-    }
+    double v[3] = {bb, rr, bs};
+    reduce_all(v, red, host);
 }
 // Fixed-order sum of the partials into out[0..2].
-__global__ void k_sum_partials(const double *part, int nb, double *out, double *host = nullptr) {
+__global__ void k_sum_partials(const double *part, int nb, double *out) {
     __shared__ double s[3][kRedThreads];
     for (int k = 0; k < 3; k++) {
         double v = 0;
@@ -1606,18 +1664,14 @@ __global__ void k_sum_partials(const double *part, int nb, double *out, double *
         __syncthreads();
     }
     if (threadIdx.x == 0)
-        for (int k = 0; k < 3; k++) {
-            out[k] = s[k][0];
-            if (host) host[k] = s[k][0];  // pinned memory: no copy behind the kernel
-        }
+        for (int k = 0; k < 3; k++) out[k] = s[k][0];
 }
 // The sums of z and b that k_norms forms of its right-hand side, by themselves
 // and in the same order: a mean needs neither the residual nor the
 // coefficients (z may be null).
-__global__ void k_sums(LevelArgs a, const double *z, const double *b, double *part) {
-    __shared__ double s1[kRedThreads], s2[kRedThreads];
+__global__ void k_sums(LevelArgs a, const double *z, const double *b, double *red) {
     double zs = 0, bs = 0;
-    const int N = a.nx * a.ny, S = gridDim.x * blockDim.x, di = S % a.nx, dj = S / a.nx;
+    const int N = a.nx * a.ny, S = kRedStride, di = S % a.nx, dj = S / a.nx;
     const int p0 = blockIdx.x * blockDim.x + threadIdx.x;
     int i = p0 % a.nx, j = p0 / a.nx;
 #pragma unroll 4
@@ -1629,18 +1683,8 @@ __global__ void k_sums(LevelArgs a, const double *z, const double *b, double *pa
         j += dj;
         if (i >= a.nx) { i -= a.nx; j++; }
     }
-    s1[threadIdx.x] = zs; s2[threadIdx.x] = bs;
-    __syncthreads();
-    for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-            s1[threadIdx.x] += s1[threadIdx.x + w];
-            s2[threadIdx.x] += s2[threadIdx.x + w];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        part[3 * blockIdx.x] = 0; part[3 * blockIdx.x + 1] = s1[0]; part[3 * blockIdx.x + 2] = s2[0];
-    }
+    double v[3] = {0, zs, bs};
+    reduce_all(v, red, nullptr);
 }
 __global__ void k_sub_means(LevelArgs a, double *z, double *b, const double *sums) {
     const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y;
@@ -1848,10 +1892,9 @@ __global__ void k_mixed_step(LevelArgs a, FemC k, const double *z, const float *
 template <int KIND>
 __global__ __launch_bounds__(kRedThreads) void k_mixed_check(LevelArgs a, FemC k, const double *z, const float *e,
                                                              const double *b, const double *c1, const double *c2,
-                                                             double *z2, float *bf, float *zf2, double *part) {
-    __shared__ double s0[kRedThreads], s1[kRedThreads];
+                                                             double *z2, float *bf, float *zf2, double *red, double *host) {
     double bb = 0, rr = 0;
-    const int N = a.nx * a.ny, S = gridDim.x * blockDim.x, di = S % a.nx, dj = S / a.nx;
+    const int N = a.nx * a.ny, S = kRedStride, di = S % a.nx, dj = S / a.nx;
     const int p0 = blockIdx.x * blockDim.x + threadIdx.x;
     int i = p0 % a.nx, j = p0 / a.nx;
 #pragma unroll 4
@@ -1864,18 +1907,8 @@ __global__ __launch_bounds__(kRedThreads) void k_mixed_check(LevelArgs a, FemC k
         j += dj;
         if (i >= a.nx) { i -= a.nx; j++; }
     }
-    s0[threadIdx.x] = bb; s1[threadIdx.x] = rr;
-    __syncthreads();
-    for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-            s0[threadIdx.x] += s0[threadIdx.x + w];
-            s1[threadIdx.x] += s1[threadIdx.x + w];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        part[3 * blockIdx.x] = s0[0]; part[3 * blockIdx.x + 1] = s1[0]; part[3 * blockIdx.x + 2] = 0;
-    }
+    double v[3] = {bb, rr, 0};
+    reduce_all(v, red, host);
 }
 __global__ void k_add_f32(LevelArgs a, double *z, const float *e) {
     const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y;
@@ -2352,7 +2385,8 @@ int Multigrid::init(MgKind kind, int m, int n, double dx, double dy, hipStream_t
     // elimination in the tail cycle), so it must be tiny
     if ((px || py || dr) && (long long)L.back().nx * L.back().ny > 16) return INCRMT_ERR_GRID;
     void *q;
-    HIP_CHECK(hipMalloc(&q, (3 * kRedBlocks + 8) * sizeof(double)));
+    HIP_CHECK(hipMalloc(&q, red_bytes()));
+    HIP_CHECK(memset_sync(q, 0, red_bytes(), s_));  // the tickets
     allocs.push_back(q);
     d_red = (double *)q;
     HIP_CHECK(hipHostMalloc((void **)&h_red, 8 * sizeof(double), hipHostMallocDefault));
@@ -3055,10 +3089,8 @@ int Multigrid::vcycle_f(size_t l) {
 
 int Multigrid::reduce_dev(double *host) {
     const MgLevel &f = L[0];
-    k_norms<<<kRedBlocks, kRedThreads, 0, s_>>>(kind_, args_of(f), fem_consts(dx_, dy_), f.z, f.b, f.fw, f.fs, f.kc,
-                                                d_red + 8);
-    KCHECK();
-    k_sum_partials<<<1, kRedThreads, 0, s_>>>(d_red + 8, kRedBlocks, d_red, host);
+    k_norms<<<red_blocks((long long)f.nx * f.ny), kRedThreads, 0, s_>>>(kind_, args_of(f), fem_consts(dx_, dy_), f.z, f.b,
+                                                                      f.fw, f.fs, f.kc, d_red, host);
     KCHECK();
     return 0;
 }
@@ -3081,14 +3113,13 @@ int Multigrid::mixed_step(bool add, double *out3) {
     const float *e = add ? f.zf : nullptr;
     float *clear = add ? f.zf2 : f.zf;
     if (out3) {
+        const int nb = red_blocks((long long)f.nx * f.ny);
         if (kind_ == kMAC)
-            k_mixed_check<kMAC><<<kRedBlocks, kRedThreads, 0, s_>>>(args_of(f), k, f.z, e, f.b, c1, c2, f.z2, f.bf, clear,
-                                                                     d_red + 8);
+            k_mixed_check<kMAC><<<nb, kRedThreads, 0, s_>>>(args_of(f), k, f.z, e, f.b, c1, c2, f.z2, f.bf, clear,
+                                                             d_red, h_red);
         else
-            k_mixed_check<kFEM><<<kRedBlocks, kRedThreads, 0, s_>>>(args_of(f), k, f.z, e, f.b, c1, c2, f.z2, f.bf, clear,
-                                                                     d_red + 8);
-        KCHECK();
-        k_sum_partials<<<1, kRedThreads, 0, s_>>>(d_red + 8, kRedBlocks, d_red, h_red);
+            k_mixed_check<kFEM><<<nb, kRedThreads, 0, s_>>>(args_of(f), k, f.z, e, f.b, c1, c2, f.z2, f.bf, clear,
+                                                             d_red, h_red);
     } else if (kind_ == kMAC) {
         k_mixed_step<kMAC><<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(args_of(f), k, f.z, e, f.b, c1, c2, f.z2, f.bf,
                                                                         clear);
@@ -3206,9 +3237,7 @@ int Multigrid::solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle, 
         // made mean-free too (the caller uses only gradients and mean-free
         // values, so the solution is unchanged)
         double *z = extrapolate ? f.z : nullptr;
-        k_sums<<<kRedBlocks, kRedThreads, 0, s_>>>(args_of(f), z, f.b, d_red + 8);
-        KCHECK();
-        k_sum_partials<<<1, kRedThreads, 0, s_>>>(d_red + 8, kRedBlocks, d_red);
+        k_sums<<<red_blocks((long long)f.nx * f.ny), kRedThreads, 0, s_>>>(args_of(f), z, f.b, d_red);
         KCHECK();
         k_sub_means<<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(args_of(f), z, f.b, d_red);
         KCHECK();
@@ -3417,9 +3446,8 @@ int Multigrid::learned_start(bool apply) {
     k_guess_apply<<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(args_of(f), f.z, dz_, d_gs_);
     KCHECK();
     if (singular()) {  // keep the start mean-free
-        k_norms<<<kRedBlocks, kRedThreads, 0, s_>>>(kind_, args_of(f), k, f.z, f.z, f.fw, f.fs, f.kc, d_red + 8);
-        KCHECK();
-        k_sum_partials<<<1, kRedThreads, 0, s_>>>(d_red + 8, kRedBlocks, d_red);
+        k_norms<<<red_blocks((long long)f.nx * f.ny), kRedThreads, 0, s_>>>(kind_, args_of(f), k, f.z, f.z, f.fw, f.fs, f.kc,
+                                                                          d_red, nullptr);
         KCHECK();
         k_sub_mean<<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(args_of(f), f.z, d_red);
         KCHECK();
