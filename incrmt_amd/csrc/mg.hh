@@ -260,8 +260,10 @@ class Multigrid {
     bool want_f32_ = false;          // a mixed solve has run: coefficient updates write FP32 copies too
     int make_f32_coefs();
     int wrap_coefs(size_t l, bool f32 = false);
-    hipGraphExec_t graph_exec_[3] = {nullptr, nullptr, nullptr};  // FP64 cycle, mixed cycle, Krylov iteration
-    std::vector<uintptr_t> graph_key_[3];                          // launch state each graph was captured in
+    // FP64 cycle, mixed cycle, Krylov iteration, a fused mixed cycle's V-cycle from either buffer
+    static constexpr int kGraphCorrection = 3, kGraphs = 5;
+    hipGraphExec_t graph_exec_[kGraphs] = {};
+    std::vector<uintptr_t> graph_key_[kGraphs];  // launch state each graph was captured in
     // Krylov solve: residual, direction, preconditioned residual, A times
     // the direction (FP64 level-0 arrays) and its device scalars
     double *kr_ = nullptr, *kp_ = nullptr, *kc_ = nullptr, *kq_ = nullptr, *ks_ = nullptr;
@@ -270,6 +272,7 @@ class Multigrid {
     std::vector<uintptr_t> launch_state() const;
     void restore_buffers(const std::vector<uintptr_t> &key);
     int run_cycle(int which, const std::function<int()> &cycle);
+    int correction_cycle();
     double *zs_ = nullptr, *dz_ = nullptr;  // learned start: the quadratic start, the network's direction
     double *eprev_ = nullptr;               // the last solve's correction to its quadratic start
     int guess_buffers();
