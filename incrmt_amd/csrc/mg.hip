@@ -945,6 +945,7 @@ template <class T>
 struct TailMac {
     T wl[2], wr[2], sd[2], su[2], d[2], y[2], b[2];
     int q[2], i[2], j;
+    int mx[2], my;  // to the points' periodic mirrors
     bool on[2], upd[2];  // on the level; updated by the sweeps (a diagonal that is not zero)
 };
 // A FEM block's: its points in colour order, the nine cells around them
@@ -952,6 +953,7 @@ template <class T>
 struct TailFem {
     T kc[9], d[4], y[4], b[4], z[4];
     int q, i, j;
+    int mx[2], my[2];  // to the mirrors of the block's columns and rows
     bool on[4], upd[4];
 };
 
@@ -983,6 +985,25 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
     auto tput = [&](const Lv &L, T *arr, int i, int j, T v) {
         if (PER) put_z(L.la, arr, i, j, v);
         else arr[j * L.v.zp + i] = v;
+    };
+    // Offsets from a point to its periodic mirrors (put_mirrors'), 0 where it has
+    // none: found once a visit, not at every write, and a mirror write is one
+    // branch (a place written twice gets the same value). With the own block's
+    // registers (off_fem) a FEM cycle of a 360^2 box takes 25.8 us instead of
+    // 32.7, a MAC cycle 21.4 instead of 22.3.
+    auto mirror_x = [&](const Lv &L, int i) -> int {
+        return PER && px && (i == 0 || i == L.v.nx - 1) ? (i == 0 ? L.v.nx : -L.v.nx) : 0;
+    };
+    auto mirror_y = [&](const Lv &L, int j) -> int {
+        return PER && py && (j == 0 || j == L.v.ny - 1) ? (j == 0 ? L.v.ny : -L.v.ny) * L.v.zp : 0;
+    };
+    auto mput = [&](T *at, int mx, int my, T v) {
+        at[0] = v;
+        if (PER && (mx | my)) {
+            at[mx] = v;
+            at[my] = v;
+            at[mx + my] = v;
+        }
     };
     // w: the first wavefront alone (lanes 0..63, wave_sync) instead of the
     // whole workgroup (__syncthreads)
@@ -1052,12 +1073,14 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
         const TailLev &v = L.v;
         const int r = (int)(((unsigned)k * v.mag) >> 20), a = k - r * v.ha;
         g.j = r;
+        g.my = mirror_y(L, r);
         const T kx = T(v.kx), ky = T(v.ky);
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             g.i[c] = 2 * a + ((c + r) & 1);
             g.on[c] = k < v.ng && g.i[c] < v.nx;
             g.q[c] = g.on[c] ? r * v.zp + g.i[c] : 0;
+            g.mx[c] = mirror_x(L, g.i[c]);
             const int q = g.q[c];
             g.wl[c] = L.c1[q]; g.wr[c] = L.c1[q + 1]; g.sd[c] = L.c2[q]; g.su[c] = L.c2[q + v.zp];
             g.b[c] = L.b[q];
@@ -1084,6 +1107,11 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
         g.i = 2 * a; g.j = 2 * r;
         g.q = mine ? g.j * v.zp + g.i : 0;
 #pragma unroll
+        for (int c = 0; c < 2; c++) {
+            g.mx[c] = mirror_x(L, g.i + c);
+            g.my[c] = mirror_y(L, g.j + c);
+        }
+#pragma unroll
         for (int c = 0; c < 9; c++) g.kc[c] = L.c1[g.q + (c / 3 - 1) * v.zp + c % 3 - 1];
 #pragma unroll
         for (int c = 0; c < 4; c++) {
@@ -1101,14 +1129,17 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
         }
         return g;
     };
-    auto off_fem = [&](const Lv &L, const TailFem<T> &g, int c) -> T {
+    auto fput = [&](const Lv &L, T *arr, const TailFem<T> &g, int c, T v) {
+        mput(arr + g.q + (c & 1) + (c >> 1) * L.v.zp, g.mx[c & 1], g.my[c >> 1], v);
+    };
+    auto off_fem = [&](const Lv &L, const TailFem<T> &g, int c, auto own) -> T {
         const int cx = c & 1, cy = c >> 1, zp = L.v.zp;
-        // a neighbour of the own block comes from its register (not on a
-        // periodic level, where a block past an odd edge holds a mirror of
-        // another block's point)
+        // own: a neighbour of the own block comes from its register (not where
+        // a periodic level may be odd, whose last block holds a mirror of
+        // another block's point: the coarsest; the others halve)
         auto nb = [&](int dx, int dy) -> T {
             const int x = cx + dx, y = cy + dy;
-            if (!PER && x >= 0 && x < 2 && y >= 0 && y < 2) return g.z[x + 2 * y];
+            if (decltype(own)::value && x >= 0 && x < 2 && y >= 0 && y < 2) return g.z[x + 2 * y];
             return L.z[g.q + x + y * zp];
         };
         const T zdl = nb(-1, -1), zdr = nb(1, -1), zul = nb(-1, 1), zur = nb(1, 1), zd = nb(0, -1), zu = nb(0, 1),
@@ -1125,6 +1156,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
     enum { kDown, kUp, kSweep };
     auto visit = [&](auto groups, auto what, const Lv &L, const Lv &C, bool w, int sweeps) {
         constexpr int G = decltype(groups)::value, WHAT = decltype(what)::value;
+        constexpr std::integral_constant<bool, !PER || WHAT != kSweep> own{};
         const int t0 = w ? lane : tid, st = w ? 64 : nt, zp = L.v.zp;
         if constexpr (KIND == kMAC) {
             TailMac<T> g[G];
@@ -1147,7 +1179,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
                             if (flip) { e2 = -e2; e22 = -e22; }
                             const T add = T(0.5625) * e[J * cz + I] + T(0.1875) * e2 + T(0.1875) * e[J2 * cz + I] +
                                           T(0.0625) * e22;
-                            tput(L, L.z, i, j, L.z[g[u].q[c]] + add);
+                            mput(L.z + g[u].q[c], g[u].mx[c], g[u].my, L.z[g[u].q[c]] + add);
                         }
                 sync(w);
             }
@@ -1162,7 +1194,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
                     for (int u = 0; u < G; u++) z[u] = quot(g[u].b[c] - off_mac(L, g[u], c), g[u].d[c], g[u].y[c]);
 #pragma unroll
                     for (int u = 0; u < G; u++)
-                        if (g[u].upd[c]) tput(L, L.z, g[u].i[c], g[u].j, z[u]);
+                        if (g[u].upd[c]) mput(L.z + g[u].q[c], g[u].mx[c], g[u].my, z[u]);
                     sync(w);
                 }
             if constexpr (WHAT == kDown) {
@@ -1202,7 +1234,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
                         for (int c = 0; c < 4; c++)
                             if (g[u].on[c]) {
                                 g[u].z[c] = g[u].z[c] + add[c];
-                                tput(L, L.z, g[u].i + (c & 1), g[u].j + (c >> 1), g[u].z[c]);
+                                fput(L, L.z, g[u], c, g[u].z[c]);
                             }
                     }
                 sync(w);
@@ -1213,12 +1245,12 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
                     const int c = WHAT == kUp ? 3 - cc : cc;
                     T z[G];
 #pragma unroll
-                    for (int u = 0; u < G; u++) z[u] = quot(g[u].b[c] - off_fem(L, g[u], c), g[u].d[c], g[u].y[c]);
+                    for (int u = 0; u < G; u++) z[u] = quot(g[u].b[c] - off_fem(L, g[u], c, own), g[u].d[c], g[u].y[c]);
 #pragma unroll
                     for (int u = 0; u < G; u++)
                         if (g[u].upd[c]) {
                             g[u].z[c] = z[u];
-                            tput(L, L.z, g[u].i + (c & 1), g[u].j + (c >> 1), z[u]);
+                            fput(L, L.z, g[u], c, z[u]);
                         }
                     sync(w);
                 }
@@ -1228,8 +1260,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
 #pragma unroll
                     for (int c = 0; c < 4; c++)
                         if (g[u].on[c])
-                            tput(L, L.c2, g[u].i + (c & 1), g[u].j + (c >> 1),
-                                 g[u].b[c] - off_fem(L, g[u], c) - g[u].d[c] * g[u].z[c]);
+                            fput(L, L.c2, g[u], c, g[u].b[c] - off_fem(L, g[u], c, own) - g[u].d[c] * g[u].z[c]);
                 sync(w);
                 const T *r = L.c2;
 #pragma unroll
