@@ -346,6 +346,10 @@ int incrmt_mg_time_solve(incrmt_mg *h, double rel_tol, int max_cycles, int preci
  * INCRMT_LAUNCH_DIRECT, default by size as for incrmt_fluid_set_launch). No
  * reference counterpart. */
 int incrmt_mg_set_launch(incrmt_mg *h, int mode);
+/* *n is the number of V-cycles this solver has captured into HIP graphs so
+ * far: one per kind of cycle and choice of iterate buffers that it has
+ * replayed. No reference counterpart. */
+int incrmt_mg_captures(incrmt_mg *h, long long *n);
 /* Mixed-precision solves (INCRMT_PREC_MIXED) as conjugate gradients in FP64
  * preconditioned by one FP32 V-cycle per iteration (on, flexible
  * Polak-Ribiere form), or as V-cycle refinement (off, the default). The

@@ -108,6 +108,7 @@ _PROTOS = [
     ("incrmt_mg_smooth", _I, [_V, _dp, _dp, _I, _I]),
     ("incrmt_mg_smooth_prec", _I, [_V, _dp, _dp, _I, _I, _I]),
     ("incrmt_mg_set_launch", _I, [_V, _I]),
+    ("incrmt_mg_captures", _I, [_V, ctypes.POINTER(ctypes.c_longlong)]),
     ("incrmt_mg_set_krylov", _I, [_V, _I]),
     ("incrmt_fluid_set_krylov", _I, [_V, _I]),
     ("incrmt_mg_time_smoother", _I, [_V, _I, _I, _dp, _ip]),
@@ -534,6 +535,13 @@ class MgSolver:
         """LAUNCH_GRAPH or LAUNCH_DIRECT V-cycles (default by size: graphs
         below 512^2 unknowns); bit-identical."""
         _check(lib().incrmt_mg_set_launch(self._h, mode))
+
+    @property
+    def captures(self):
+        """V-cycles captured into HIP graphs so far."""
+        n = ctypes.c_longlong(0)
+        _check(lib().incrmt_mg_captures(self._h, ctypes.byref(n)))
+        return n.value
 
     def set_krylov(self, on):
         """Mixed-precision solves as FP64 conjugate gradients preconditioned

@@ -1686,6 +1686,12 @@ int incrmt_mg_set_launch(incrmt_mg *h, int mode) {
     return 0;
 }
 
+int incrmt_mg_captures(incrmt_mg *h, long long *n) {
+    if (!h || !n) return fail(INCRMT_ERR_ARG, "null argument");
+    *n = h->mg.captures;
+    return 0;
+}
+
 int incrmt_mg_smooth(incrmt_mg *h, const double *b, double *z, int sweeps, int shape) {
     return incrmt_mg_smooth_prec(h, b, z, sweeps, shape, INCRMT_PREC_FP64);
 }

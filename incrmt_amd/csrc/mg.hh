@@ -240,6 +240,7 @@ class Multigrid {
     // sets it for hierarchies whose finest level is below kGraphMaxPoints
     bool use_graphs = true;
     static constexpr long long kGraphMaxPoints = 512LL * 512;
+    long captures = 0;  // V-cycles captured so far
     double smoother_ms = 0;
     long smoother_launches = 0;
     double smoother_bytes = 0;  // algorithmic bytes of the timed sweeps
@@ -260,19 +261,21 @@ class Multigrid {
     bool want_f32_ = false;          // a mixed solve has run: coefficient updates write FP32 copies too
     int make_f32_coefs();
     int wrap_coefs(size_t l, bool f32 = false);
-    // FP64 cycle, mixed cycle, Krylov iteration, a fused mixed cycle's V-cycle from either buffer
-    static constexpr int kGraphCorrection = 3, kGraphs = 5;
-    hipGraphExec_t graph_exec_[kGraphs] = {};
-    std::vector<uintptr_t> graph_key_[kGraphs];  // launch state each graph was captured in
+    // what a captured cycle does; kCorrection: the V-cycle alone of a mixed
+    // cycle whose update and residual go together (mixed_step)
+    enum CycleKind { kCycle64, kCycleMixed, kCycleKrylov, kCorrection, kCycleKinds };
+    // a graph per kind and choice of level 0's current buffers (FP64, FP32)
+    hipGraphExec_t graph_exec_[kCycleKinds][4] = {};
+    std::vector<uintptr_t> graph_key_[kCycleKinds][4];  // launch state each graph was captured in
     // Krylov solve: residual, direction, preconditioned residual, A times
     // the direction (FP64 level-0 arrays) and its device scalars
     double *kr_ = nullptr, *kp_ = nullptr, *kc_ = nullptr, *kq_ = nullptr, *ks_ = nullptr;
     int krylov_buffers();
     int solve_krylov(double tol, int max_cycles, MgStats *st);
-    std::vector<uintptr_t> launch_state() const;
-    void restore_buffers(const std::vector<uintptr_t> &key);
-    int run_cycle(int which, const std::function<int()> &cycle);
-    int correction_cycle();
+    std::vector<uintptr_t> launch_state(CycleKind kind) const;
+    std::vector<uintptr_t> buffers() const;
+    void restore_buffers(const std::vector<uintptr_t> &was);
+    int run_cycle(CycleKind kind, const std::function<int()> &cycle);
     double *zs_ = nullptr, *dz_ = nullptr;  // learned start: the quadratic start, the network's direction
     double *eprev_ = nullptr;               // the last solve's correction to its quadratic start
     int guess_buffers();

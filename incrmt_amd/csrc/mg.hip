@@ -2301,8 +2301,9 @@ int Multigrid::tail_coefs(bool f32, bool copy) {
 }
 
 Multigrid::~Multigrid() {
-    for (auto &g : graph_exec_)
-        if (g) (void)hipGraphExecDestroy(g);
+    for (auto &kind : graph_exec_)
+        for (auto &g : kind)
+            if (g) (void)hipGraphExecDestroy(g);
     for (auto &e : ev_) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
     for (hipEvent_t e : cev_)
         if (e) (void)hipEventDestroy(e);
@@ -3373,11 +3374,11 @@ int Multigrid::solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle, 
     double rel = bn > 0 ? std::sqrt(nr[1]) / bn : 0;
     int cycles = 0;
     bool fallback = false;
-    auto fp64_cycle = [&]() -> int { return run_cycle(0, [&]() { return vcycle(0); }); };
+    auto fp64_cycle = [&]() -> int { return run_cycle(kCycle64, [&]() { return vcycle(0); }); };
     // one cycle, and a check of the residual behind it
     auto next = [&](bool check) -> int {
         if (fused) {
-            if (int e = correction_cycle()) return e;
+            if (int e = run_cycle(kCorrection, [&]() { return vcycle_f(0); })) return e;
             return mixed_step(true, check ? nr : nullptr);
         }
         if (int e = fallback ? fp64_cycle() : cycle()) return e;
@@ -3441,79 +3442,85 @@ int Multigrid::solve_loop(double tol, int max_cycles, MgStats *st, Cycle cycle, 
 // One V-cycle as a HIP graph. A cycle's launch sequence is fixed by the
 // hierarchy (kernels, launch shapes, sweep counts) and by which of each
 // level's two iterate buffers is current, so it is captured once and
-// replayed while those stay the same; a smoothing or timing call between
-// solves that leaves the other buffer current makes the next solve capture
-// again. Each level's fused smoother swaps its buffers an even number of
-// times per cycle (as many pre- as post-smoothing launches), so a cycle ends
-// in the buffer state it began in; a hierarchy where that fails launches its
-// cycles directly. Nothing in a cycle sets memory with a memset node (every
-// array a cycle clears is cleared by a kernel), and timing runs (HIP events
-// around smoother launches) always launch directly.
-std::vector<uintptr_t> Multigrid::launch_state() const {
+// replayed while those stay the same. Level 0's buffers change between solves
+// (a smoothing or timing call with an odd number of launches, an odd number of
+// mixed cycles whose updates go from one buffer to the other) and between the
+// cycles of one solve (those updates), so a graph is kept for each choice of
+// the buffers that its kind of cycle uses: whatever is called in between, each
+// is captured once. Within a cycle each level's fused smoother swaps its
+// buffers an even number of times (as many pre- as post-smoothing launches),
+// so a cycle ends in the buffer state it began in; a hierarchy where that
+// fails launches its cycles directly. Nothing in a cycle sets memory with a
+// memset node (every array a cycle clears is cleared by a kernel), and timing
+// runs (HIP events around smoother launches) always launch directly.
+std::vector<uintptr_t> Multigrid::launch_state(CycleKind kind) const {
     std::vector<uintptr_t> k{(uintptr_t)nu1, (uintptr_t)nu2, (uintptr_t)tail_};
+    // the FP32 cycles leave the FP64 buffers alone, but for level 0's
+    // iterate where the update belongs to the cycle
+    if (kind == kCycleMixed || kind == kCycleKrylov) k.push_back((uintptr_t)L[0].z);
     for (const MgLevel &v : L) {
-        k.insert(k.end(), {(uintptr_t)v.z, (uintptr_t)v.z2, (uintptr_t)v.zf, (uintptr_t)v.zf2});
-        k.insert(k.end(), {(uintptr_t)v.shape64, (uintptr_t)v.shape32});
+        if (kind == kCycle64) k.insert(k.end(), {(uintptr_t)v.z, (uintptr_t)v.z2, (uintptr_t)v.shape64});
+        else k.insert(k.end(), {(uintptr_t)v.zf, (uintptr_t)v.zf2, (uintptr_t)v.shape32});
     }
     return k;
 }
 
-void Multigrid::restore_buffers(const std::vector<uintptr_t> &key) {
-    size_t i = 3;
+std::vector<uintptr_t> Multigrid::buffers() const {
+    std::vector<uintptr_t> k;
+    for (const MgLevel &v : L) k.insert(k.end(), {(uintptr_t)v.z, (uintptr_t)v.z2, (uintptr_t)v.zf, (uintptr_t)v.zf2});
+    return k;
+}
+
+void Multigrid::restore_buffers(const std::vector<uintptr_t> &was) {
+    size_t i = 0;
     for (MgLevel &v : L) {
-        v.z = (double *)key[i]; v.z2 = (double *)key[i + 1];
-        v.zf = (float *)key[i + 2]; v.zf2 = (float *)key[i + 3];
-        i += 6;
+        v.z = (double *)was[i]; v.z2 = (double *)was[i + 1];
+        v.zf = (float *)was[i + 2]; v.zf2 = (float *)was[i + 3];
+        i += 4;
     }
 }
 
-int Multigrid::run_cycle(int which, const std::function<int()> &cycle) {
+int Multigrid::run_cycle(CycleKind kind, const std::function<int()> &cycle) {
     if (!use_graphs || time_smoother) return cycle();
-    const std::vector<uintptr_t> key = launch_state();
-    if (graph_exec_[which] && graph_key_[which] != key) {
-        (void)hipGraphExecDestroy(graph_exec_[which]);
-        graph_exec_[which] = nullptr;
+    const std::vector<uintptr_t> key = launch_state(kind);
+    const int slot = (kind != kCorrection && L[0].z > L[0].z2) + 2 * (kind != kCycle64 && L[0].zf > L[0].zf2);
+    hipGraphExec_t &exec = graph_exec_[kind][slot];
+    if (exec && graph_key_[kind][slot] != key) {
+        // (its last replay may still run: cycles are not waited for one by one)
+        HIP_CHECK(hipStreamSynchronize(s_));
+        (void)hipGraphExecDestroy(exec);
+        exec = nullptr;
     }
-    if (!graph_exec_[which]) {
+    if (!exec) {
+        const std::vector<uintptr_t> was = buffers();
         hipGraph_t g = nullptr;
         HIP_CHECK(hipStreamBeginCapture(s_, hipStreamCaptureModeThreadLocal));
         const int rc = cycle();
         const hipError_t e = hipStreamEndCapture(s_, &g);
         if (rc || e != hipSuccess) {
             if (g) (void)hipGraphDestroy(g);
-            restore_buffers(key);  // nothing ran
+            restore_buffers(was);  // nothing ran
             return rc ? rc : hip_fail(e, "hipStreamEndCapture", __FILE__, __LINE__);
         }
-        if (launch_state() != key) {
+        if (buffers() != was) {
             // the cycle leaves other buffers current: a replay would start
             // from the wrong ones, so this hierarchy launches directly
             (void)hipGraphDestroy(g);
-            restore_buffers(key);
+            restore_buffers(was);
             use_graphs = false;
             return cycle();
         }
-        const hipError_t e2 = hipGraphInstantiate(&graph_exec_[which], g, nullptr, nullptr, 0);
+        const hipError_t e2 = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         if (e2 != hipSuccess) {
-            graph_exec_[which] = nullptr;
+            exec = nullptr;
             return hip_fail(e2, "hipGraphInstantiate", __FILE__, __LINE__);
         }
-        graph_key_[which] = key;
+        graph_key_[kind][slot] = key;
+        captures++;
     }
-    HIP_CHECK(hipGraphLaunch(graph_exec_[which], s_));
+    HIP_CHECK(hipGraphLaunch(exec, s_));
     return 0;
-}
-
-// A mixed cycle's V-cycle. Its iterate is in either buffer in turn
-// (mixed_step), so there are two graphs, found by the state they replay from.
-int Multigrid::correction_cycle() {
-    int slot = kGraphCorrection;
-    if (use_graphs) {
-        const std::vector<uintptr_t> key = launch_state();
-        const auto holds = [&](int k) { return graph_exec_[k] && graph_key_[k] == key; };
-        if (!holds(slot) && (holds(slot + 1) || (graph_exec_[slot] && !graph_exec_[slot + 1]))) slot++;
-    }
-    return run_cycle(slot, [&]() { return vcycle_f(0); });
 }
 
 int Multigrid::guess_buffers() {
@@ -3603,7 +3610,7 @@ void Multigrid::set_extrapolate(int mode) {
 }
 
 int Multigrid::solve(double tol, int max_cycles, MgStats *st) {
-    return solve_loop(tol, max_cycles, st, [&]() { return run_cycle(0, [&]() { return vcycle(0); }); });
+    return solve_loop(tol, max_cycles, st, [&]() { return run_cycle(kCycle64, [&]() { return vcycle(0); }); });
 }
 
 int Multigrid::krylov_buffers() {
@@ -3642,7 +3649,7 @@ int Multigrid::solve_krylov(double tol, int max_cycles, MgStats *st) {
             KCHECK();
             started = true;
         }
-        return run_cycle(2, [&]() -> int {
+        return run_cycle(kCycleKrylov, [&]() -> int {
             const MgLevel &g = L[0];
             const LevelArgs a = args_of(g);
             if (int rc = vcycle_f(0)) return rc;
@@ -3682,7 +3689,7 @@ int Multigrid::solve_mixed(double tol, int max_cycles, MgStats *st) {
     const bool fused = !f.px && !f.py && !net;
     // FP64 residual -> FP32 right-hand side, FP32 V-cycle, FP64 update
     return solve_loop(tol, max_cycles, st, [&]() -> int {
-        return run_cycle(1, [&]() -> int {
+        return run_cycle(kCycleMixed, [&]() -> int {
             k_residual_f32<<<grid2(f.nx, f.ny), dim3(BX, BY), 0, s_>>>(kind_, args_of(f), k, f.z, f.b, f.fw, f.fs,
                                                                         f.kc, f.bf, f.zf);
             KCHECK();
