@@ -16,6 +16,7 @@
 #include <type_traits>
 #include <hip/hip_ext.h>
 #include "mg.hh"
+#include "quot.hh"
 #include "unet.hh"
 
 namespace incrmt {
@@ -916,21 +917,6 @@ __device__ double tail_block_sum(double v, double *red) {
 // (a fence would wait for every write's end, 100 cycles a phase)
 __device__ inline void wave_sync() { asm volatile("" ::: "memory"); }
 
-// n / d, correctly rounded, from y = 1 / d correctly rounded (P. Markstein,
-// IBM J. Res. Dev. 34, 1990: with q within a rounding of n / d, the remainder
-// n - d q is exact in one fused operation and q + y (n - d q) rounds to the
-// quotient; the first correction brings q there). Five dependent operations
-// instead of a division's thirty.
-__host__ __device__ inline double quot(double n, double d, double y) {
-    double q = n * y;
-    q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
-    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
-}
-__host__ __device__ inline float quot(float n, float d, float y) {
-    float q = n * y;
-    q = __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
-    return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
-}
 __device__ inline double read_lane(double v, int l) {
     const unsigned long long b = (unsigned long long)__double_as_longlong(v);
     const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, l), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), l);
@@ -1191,7 +1177,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
                     // two groups' chains overlap)
                     T z[G];
 #pragma unroll
-                    for (int u = 0; u < G; u++) z[u] = quot(g[u].b[c] - off_mac(L, g[u], c), g[u].d[c], g[u].y[c]);
+                    for (int u = 0; u < G; u++) z[u] = quot<false>(g[u].b[c] - off_mac(L, g[u], c), g[u].d[c], g[u].y[c]);
 #pragma unroll
                     for (int u = 0; u < G; u++)
                         if (g[u].upd[c]) mput(L.z + g[u].q[c], g[u].mx[c], g[u].my, z[u]);
@@ -1245,7 +1231,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
                     const int c = WHAT == kUp ? 3 - cc : cc;
                     T z[G];
 #pragma unroll
-                    for (int u = 0; u < G; u++) z[u] = quot(g[u].b[c] - off_fem(L, g[u], c, own), g[u].d[c], g[u].y[c]);
+                    for (int u = 0; u < G; u++) z[u] = quot<true>(g[u].b[c] - off_fem(L, g[u], c, own), g[u].d[c], g[u].y[c]);
 #pragma unroll
                     for (int u = 0; u < G; u++)
                         if (g[u].upd[c]) {
@@ -1319,7 +1305,7 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
             T acc = 0;
 #pragma unroll
             for (int c = k + 1; c < M; c++) acc += row[c] * xs[c];
-            const T xk = quot(rhs - acc, piv, y);
+            const T xk = quot<KIND == kFEM>(rhs - acc, piv, y);
             if (r == k && solved) x = xk;
             xs[k] = k < n ? read_lane(xk, k + o) : T(0);
         }
