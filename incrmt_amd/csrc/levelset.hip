@@ -811,9 +811,30 @@ __global__ void k_commit_status(Grid g, ObjArrays a, LsWork w, Win wn) { commit_
 // -> 0.12 ms against 14 to 20 launches that swept whole tiles to a local fixed
 // point (25-31 us each); 64 circles at 2048^2 3.3 -> 0.75 ms. At 64^2 about 26
 // of the 64 links cross between workgroups.
-constexpr int kEH = 3, kEW = kTileX + 2 * kEH, kEHt = kTileY + 2 * kEH, kEN = kEW * kEHt;
-static_assert(kEW <= 32, "a row of the tile and its halo is one 32-bit word of flags");
-constexpr int kExtWaves = kTileThreads / 64, kExtThreads = kTileThreads + 64;
+constexpr int kEH = 3;
+// Its tiles are the march's, whole where a row with its halo fits one 32-bit word
+// of flags and the points' wavefronts and one more a workgroup (the default
+// 16 x 16 does), else in the fewest equal parts of whole wavefronts for which
+// that holds.
+struct ExtParts {
+    int x = 0, y = 0;
+};
+constexpr ExtParts ext_parts(int tx, int ty) {
+    ExtParts best;
+    for (int x = 1; x <= tx; x++)
+        for (int y = 1; y <= ty; y++) {
+            const int ex = tx / x, ey = ty / y;
+            if (tx % x || ty % y || ex + 2 * kEH > 32 || ex * ey % 64 || ex * ey + 64 > 1024) continue;
+            if (!best.x || x * y < best.x * best.y) best = {x, y};
+        }
+    return best;
+}
+constexpr ExtParts kExtParts = ext_parts(kTileX, kTileY);
+static_assert(kExtParts.x > 0, "the extension needs parts of whole wavefronts, at most 26 points wide");
+constexpr int kExtPerTile = kExtParts.x * kExtParts.y;
+constexpr int kExtX = kTileX / kExtParts.x, kExtY = kTileY / kExtParts.y;
+constexpr int kEW = kExtX + 2 * kEH, kEHt = kExtY + 2 * kEH, kEN = kEW * kEHt;
+constexpr int kExtWaves = kExtX * kExtY / 64, kExtThreads = kExtX * kExtY + 64;
 // a signalling NaN, which no arithmetic returns
 constexpr unsigned long long kExtOpen = 0x7ff4a5a5a5a5a5a5ull;
 constexpr int kExtProd = 49;  // row of products: at most 48 neighbours; odd, so that six rows start in different banks
@@ -871,9 +892,10 @@ struct ExtLds {
 // k_ext_open left it (the first visit of the first pass). Returns the points
 // still open.
 __device__ __forceinline__ int extend_tile(const Grid &g, const ObjArrays &a, const LsWork &w, ExtLds &L, int tile,
-                                           bool fresh, int patience) {
+                                           int part, bool fresh, int patience) {
     const int m = g.ml, nn = g.nl, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int I0 = tile % w.ntx * kTileX - kEH, J0 = tile / w.ntx * kTileY - kEH;
+    const int I0 = tile % w.ntx * kTileX + part % kExtParts.x * kExtX - kEH,
+              J0 = tile / w.ntx * kTileY + part / kExtParts.x * kExtY - kEH;
     // the tile and its halo, two rows a wavefront: every global read issued
     // before any wait, both rows' flags from one ballot
     constexpr int kRowsAtOnce = kExtThreads / 32, kRounds = (kEHt + kRowsAtOnce - 1) / kRowsAtOnce;
@@ -911,7 +933,7 @@ __device__ __forceinline__ int extend_tile(const Grid &g, const ObjArrays &a, co
         }
     }
     __syncthreads();
-    const int li = tid % kTileX + kEH, lj = tid / kTileX + kEH, e = lj * kEW + li;
+    const int li = tid % kExtX + kEH, lj = tid / kExtX + kEH, e = lj * kEW + li;
     const int i = I0 + li, j = J0 + lj;
     const bool mine = wave < kExtWaves && i < m && j < nn && (L.st[e] == 5 || L.st[e] == 6);
     const int q = mine ? g.ls(i, j) : 0;
@@ -1020,7 +1042,7 @@ __device__ __forceinline__ int extend_tile(const Grid &g, const ObjArrays &a, co
     if (lane == 0 && open) atomicAdd(&L.left, __popcll(open));
     __syncthreads();
     if (tid < kEHt) {  // the halo points to poll, a row a thread
-        const unsigned own = tid >= kEH && tid < kEH + kTileY ? ((1u << kTileX) - 1) << kEH : 0u;
+        const unsigned own = tid >= kEH && tid < kEH + kExtY ? ((1u << kExtX) - 1) << kEH : 0u;
         unsigned b = L.need[tid] & ~L.known[tid] & ~own;
         int at = b ? atomicAdd(&L.nhalo, __popc(b)) : 0;
         for (; b; b &= b - 1) L.halo[at++] = (unsigned short)(tid * kEW + __ffs(b) - 1);
@@ -1034,7 +1056,7 @@ __device__ __forceinline__ int extend_tile(const Grid &g, const ObjArrays &a, co
         // each lane keeps its points of the list in registers: a poll is
         // their two loads (0.1 us where the line is in the L2 and nothing
         // has come; a value takes 0.6-0.8 us from store to here)
-        constexpr int kOwn = (kEN - kTileThreads + 63) / 64;
+        constexpr int kOwn = (kEN - kExtX * kExtY + 63) / 64;
         int at[kOwn], hp[kOwn];
 #pragma unroll
         for (int u = 0; u < kOwn; u++) {
@@ -1222,7 +1244,7 @@ constexpr int kPatienceMany = 16, kPatienceLast = 2000, kExtRounds = 64;
 __device__ __forceinline__ void extend_tiles(const Grid &g, const ObjArrays &a, const LsWork &w, int p, int slot) {
     __shared__ ExtLds L;
     if (slot > 0 && w.cnt[kCntIter + slot - 1] == 0) return;  // nothing left open
-    const int nt = w.cnt[kCntTileExt];
+    const int nt = w.cnt[kCntTileExt] * kExtPerTile;
     unsigned long long done = 0;  // of the block's first 64 tiles
     int open = 0;
     for (int round = 0; round < kExtRounds; round++) {
@@ -1234,8 +1256,8 @@ __device__ __forceinline__ void extend_tiles(const Grid &g, const ObjArrays &a, 
         one = left == 1;
         for (int t = blockIdx.x, k = 0; t < nt; t += gridDim.x, k++) {
             if (k < 64 && (done >> k & 1)) continue;
-            const int still = extend_tile(g, a, w, L, w.tiles_ext[t], p == 0 && round == 0,
-                                          one ? kPatienceLast : kPatienceMany);
+            const int still = extend_tile(g, a, w, L, w.tiles_ext[t / kExtPerTile], t % kExtPerTile,
+                                          p == 0 && round == 0, one ? kPatienceLast : kPatienceMany);
             if (still) open++;
             else if (k < 64) done |= 1ull << k;
         }
