@@ -9,9 +9,10 @@
 
 namespace incrmt {
 
-// Counter slots in LsWork::cnt
-enum { kCntIface = 0, kCntErr, kCntTileFim, kCntTileExt, kCntIter };
+// Counter slots in LsWork::cnt; from kCntTicket and from kCntIter one for each
+// pass of a batch: the extension's tickets, what a pass left to do
 constexpr int kIterSlots = 64;
+enum { kCntIface = 0, kCntErr, kCntTileFim, kCntTileExt, kCntExtMoved, kCntTicket, kCntIter = kCntTicket + kIterSlots };
 enum { kErrNewton = 1, kErrSingular = 2 };
 
 // The fixed-point passes run on kTileX x kTileY tiles of the ghosted grid
@@ -33,6 +34,7 @@ struct LsWork {
     unsigned char *cflag; // 1 where a point takes part in the march
     int *tflag;           // per-tile flags: bit 1 march, bit 2 extension
     int *tiles_fim, *tiles_ext;  // active tile lists
+    int *tprog;           // per tile: batches of points the extension has evaluated
     int ntx, nty;         // tile grid
     int *cnt;             // counters (kCntIter + kIterSlots ints)
     int *hcnt;            // pinned host mirror

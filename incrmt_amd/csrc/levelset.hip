@@ -801,11 +801,11 @@ __global__ void k_commit_status(Grid g, ObjArrays a, LsWork w, Win wn) { commit_
 // its tile's open points read. A value is its own flag, so nothing is fenced.
 // No barrier, launch or host check lies between two links.
 //
-// A tile whose halo brings nothing new for its patience is left: the block
-// goes on to its other tiles and comes back, and what is still open at the
-// end is counted for another pass, which takes up the values found so far.
-// So the kernel ends whatever the other workgroups do, also when not all of
-// them are on the GPU at once.
+// A tile whose halo brings nothing new for its patience is left: the workgroup
+// takes or goes on to others and comes back (ext_next), and what is still open
+// when nothing moves any more is counted for another pass, which takes up the
+// values found so far. So the kernel ends whatever the other workgroups do,
+// also when not all of them are on the GPU at once.
 //
 // Measured per extension: a rotor at 64^2 0.63 -> 0.09 ms and at 1024^2 0.44
 // -> 0.12 ms against 14 to 20 launches that swept whole tiles to a local fixed
@@ -861,11 +861,12 @@ __device__ __forceinline__ double lane_double(double v, int l) {
     return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
 
-// Mark the outside band points of the active tiles open.
+// Mark the outside band points of the active tiles open, clear the tiles' counters.
 __device__ __forceinline__ void ext_open_body(const Grid &g, const ObjArrays &a, const LsWork &w) {
     const int nt = w.cnt[kCntTileExt];
     for (int t = blockIdx.x; t < nt; t += gridDim.x) {
         const int tile = w.tiles_ext[t];
+        if (threadIdx.x == 0) w.tprog[tile] = 0;
         const int I = tile % w.ntx * kTileX + threadIdx.x % kTileX, J = tile / w.ntx * kTileY + threadIdx.x / kTileX;
         if (I >= g.ml || J >= g.nl) continue;
         const int q = g.ls(I, J), s = a.st[q];
@@ -877,6 +878,7 @@ __device__ __forceinline__ void ext_open_body(const Grid &g, const ObjArrays &a,
 }
 __global__ __launch_bounds__(kTileThreads) void k_ext_open(Grid g, ObjArrays a, LsWork w) { ext_open_body(g, a, w); }
 
+constexpr int kExtHeld = 32;  // tiles that a workgroup goes round between at the most
 struct ExtLds {
     double phi[kEN], x[kEN], y[kEN];
     double prod[kExtWaves][6][kExtProd];
@@ -886,13 +888,40 @@ struct ExtLds {
     unsigned short halo[kEN];        // the halo points to poll
     int nhalo, left, stop;
     unsigned news;                   // counts values that have become final here
+    int was;                         // points open before the visit
+    // ext_next's state: the visit (tile number, -1: none; its place in held,
+    // ext_news before it), the tiles held and ext_news before their last
+    // visits (-1: none yet)
+    int t, k, heard, patience, nheld, open, idle, moved;
+    bool fresh, more, take;
+    int held[kExtHeld], seen[kExtHeld];
 };
 
+// Rounds of idle polling (0.2-1 us each) before a tile is left. kPatienceMany: by
+// a workgroup that holds others too (the lattice of 6924 tiles 2.1, 2.1 and 3.0 ms for
+// 8, 16 and 64). kPatienceTake: by one that holds this tile only and may take
+// another, which workgroups that have finished should do first (32, 64, 128, 256, 512,
+// 1024: a lattice of 1000 tiles 270, 250, 165, 175, 185, 180 us, that of 6924 2.2, 2.2,
+// 2.2, 2.4, 2.7, 3.1 ms). kPatienceLast: where no other is to be had; then again
+// while any of the solid's tiles has moved since, which a tile tells every
+// kTellPoints points (without that 64 circles on 2048^2 took two launches with 200, one
+// with 2000).
+constexpr int kPatienceMany = 16, kPatienceTake = 256, kPatienceLast = 1000, kTellPoints = 32;
+// Fruitless looks (1-2 us each) at the tiles of a workgroup that holds several
+// before it asks the same, and leaves them to another pass
+constexpr int kIdleMany = 256;
+__device__ __forceinline__ void ext_tell(const LsWork &w) {
+    (void)__hip_atomic_fetch_add(&w.cnt[kCntExtMoved], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int ext_moved(const LsWork &w) {
+    return __hip_atomic_load(&w.cnt[kCntExtMoved], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // One visit of a tile. fresh: every open mark of this extension is still as
-// k_ext_open left it (the first visit of the first pass). Returns the points
-// still open.
-__device__ __forceinline__ int extend_tile(const Grid &g, const ObjArrays &a, const LsWork &w, ExtLds &L, int tile,
-                                           int part, bool fresh, int patience) {
+// k_ext_open left it (the first visit of the first pass); many: the tile's counter
+// is kept for ext_news. L.was and L.left: the points open before and after it.
+__device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, const LsWork &w, ExtLds &L, int tile,
+                                           int part, bool fresh, bool many, int patience) {
     const int m = g.ml, nn = g.nl, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int I0 = tile % w.ntx * kTileX + part % kExtParts.x * kExtX - kEH,
               J0 = tile / w.ntx * kTileY + part / kExtParts.x * kExtY - kEH;
@@ -1041,6 +1070,7 @@ __device__ __forceinline__ int extend_tile(const Grid &g, const ObjArrays &a, co
     const unsigned long long open = __ballot(todo);
     if (lane == 0 && open) atomicAdd(&L.left, __popcll(open));
     __syncthreads();
+    if (tid == 0) L.was = L.left;
     if (tid < kEHt) {  // the halo points to poll, a row a thread
         const unsigned own = tid >= kEH && tid < kEH + kExtY ? ((1u << kExtX) - 1) << kEH : 0u;
         unsigned b = L.need[tid] & ~L.known[tid] & ~own;
@@ -1064,7 +1094,7 @@ __device__ __forceinline__ int extend_tile(const Grid &g, const ObjArrays &a, co
             hp[u] = k < nh ? L.halo[k] : -1;
             at[u] = hp[u] < 0 ? 0 : g.ls(I0 + hp[u] % kEW, J0 + hp[u] / kEW);
         }
-        int seen = -1, idle = 0;
+        int seen = -1, idle = 0, moved = -1;
         while (true) {
             unsigned long long px[kOwn], py[kOwn];
 #pragma unroll
@@ -1089,11 +1119,17 @@ __device__ __forceinline__ int extend_tile(const Grid &g, const ObjArrays &a, co
             const int lf = lds_now(L.left);
             if (lf == 0) break;
             if (lf != seen || any) {
+                if (((lf ^ seen) & -kTellPoints) && lane == 0) ext_tell(w);
                 seen = lf;
                 idle = 0;
             } else if (++idle > patience) {
-                if (lane == 0) atomicOr(&L.stop, 1);
-                break;
+                const int now = patience == kPatienceLast ? ext_moved(w) : moved;
+                if (now == moved) {
+                    if (lane == 0) atomicOr(&L.stop, 1);
+                    break;
+                }
+                moved = now;
+                idle = 0;
             }
             if (!nh) __builtin_amdgcn_s_sleep(8);
         }
@@ -1228,42 +1264,144 @@ __device__ __forceinline__ int extend_tile(const Grid &g, const ObjArrays &a, co
                 }
             }
             if (lane == 0) atomicSub(&L.left, __popcll(rd));
+            if (many && lane == 0) (void)__hip_atomic_fetch_add(&w.tprog[tile], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     __syncthreads();
-    const int still = L.left;
-    __syncthreads();
-    return still;
 }
 
-// Rounds of idle polling (0.2-1 us each) before a tile is left: few while
-// the block has other open tiles, many for its last one, which waits for a
-// chain through other workgroups' tiles.
-constexpr int kPatienceMany = 16, kPatienceLast = 2000, kExtRounds = 64;
+// Tiles that hold what a part of a tile reads, to either side (fits reach 7 points)
+constexpr int kNewsX = (7 + kTileX - 1) / kTileX, kNewsY = (7 + kTileY - 1) / kTileY;
+static_assert((2 * kNewsX + 1) * (2 * kNewsY + 1) <= 64, "a lane a tile");
+// The sum of those tiles' counters of evaluated batches (its own tile's only where
+// that has other parts): where it stays, a visit would find what the last one left.
+// For a whole wavefront.
+__device__ __forceinline__ int ext_news(const LsWork &w, int tile) {
+    const int lane = __lane_id(), dx = lane % (2 * kNewsX + 1) - kNewsX, dy = lane / (2 * kNewsX + 1) - kNewsY;
+    const int X = tile % w.ntx + dx, Y = tile / w.ntx + dy;
+    int n = 0;
+    if (dy <= kNewsY && X >= 0 && X < w.ntx && Y >= 0 && Y < w.nty && (kExtPerTile > 1 || dx || dy))
+        n = __hip_atomic_load(&w.tprog[tile + dy * w.ntx + dx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int h = 32; h > 0; h /= 2) n += __shfl_xor(n, h, 64);
+    return n;
+}
+
+// The workgroup's next visit, by its first wavefront. A workgroup takes one tile
+// and, while there are others that nobody has, a further one whenever a look at
+// all it holds brought nothing: so a tile that others wait for is held by a
+// workgroup that runs, however many there are. It visits a tile again when
+// ext_news has changed. (With the tiles dealt out beforehand and visited in turn,
+// news or not, a band 200 cells wide on 1400^2, 2963 tiles, took 700 to 1040 ms, now
+// 9; a lattice of blobs, 6924 tiles, 12.5 to 14, now 2.4.)
+__device__ __forceinline__ void ext_next(const LsWork &w, ExtLds &L, int nt, int p, int slot) {
+    const bool first = __lane_id() == 0;
+    int k = L.k, held = L.nheld, idle = L.idle;
+    bool more = L.more, take = L.take;
+    auto go = [&](int t, int news, bool fresh, int patience) {
+        if (!first) return;
+        L.t = t; L.k = k; L.heard = news; L.fresh = fresh; L.patience = patience;
+        L.nheld = held; L.idle = idle; L.more = more; L.take = take;
+    };
+    auto end = [&]() {
+        if (L.open + held && first) atomicAdd(&w.cnt[kCntIter + slot], L.open + held);
+        go(-1, 0, false, 0);
+    };
+    // the visit that has ended
+    const int left = L.left;
+    if (left < L.was) {
+        idle = 0;
+        take = false;
+        if (first) ext_tell(w);
+    } else {
+        idle += kPatienceMany;
+    }
+    if (left) {
+        if (first) L.seen[k] = L.heard;
+        k++;
+    } else {  // the last one takes its place
+        held--;
+        if (first) {
+            L.held[k] = L.held[held];
+            L.seen[k] = L.seen[held];
+        }
+    }
+    lds_order();
+    // the last of all was waited for as long as anything moved
+    if (L.patience == kPatienceLast) return end();
+    while (true) {
+        const bool one = held == 1 && !more;
+        for (; k < held; k++) {
+            const int t = L.held[k], seen = L.seen[k];
+            const int news = ext_news(w, w.tiles_ext[t / kExtPerTile]);
+            if (seen != news || one)
+                return go(t, news, p == 0 && seen == -1, one ? kPatienceLast : held == 1 ? kPatienceTake : kPatienceMany);
+            idle++;
+        }
+        // all looked at
+        if (idle > kIdleMany) {  // nothing for long: stay while any of the solid's tiles moves
+            const int now = ext_moved(w);
+            if (now == L.moved) {
+                if (first) L.open += held;
+                held = 0;
+            } else if (first) {
+                L.moved = now;
+            }
+            lds_order();
+            idle = 0;
+        }
+        if (more && (take || !held) && held < kExtHeld) {
+            int t = 0;
+            if (first) t = gridDim.x + atomicAdd(&w.cnt[kCntTicket + slot], 1);
+            t = __builtin_amdgcn_readfirstlane(t);
+            more = t < nt;
+            if (more) {
+                if (first) {
+                    L.held[held] = t;
+                    L.seen[held] = -1;
+                }
+                held++;
+                lds_order();
+            }
+        }
+        if (!held && !more) return end();
+        k = 0;
+        take = true;
+    }
+}
 
 __device__ __forceinline__ void extend_tiles(const Grid &g, const ObjArrays &a, const LsWork &w, int p, int slot) {
     __shared__ ExtLds L;
     if (slot > 0 && w.cnt[kCntIter + slot - 1] == 0) return;  // nothing left open
     const int nt = w.cnt[kCntTileExt] * kExtPerTile;
-    unsigned long long done = 0;  // of the block's first 64 tiles
-    int open = 0;
-    for (int round = 0; round < kExtRounds; round++) {
-        open = 0;
-        bool one = false;  // a single tile was left by the last round, or there is one at all
-        int left = 0;
-        for (int t = blockIdx.x, k = 0; t < nt; t += gridDim.x, k++) left += !(k < 64 && (done >> k & 1));
-        if (!left) break;
-        one = left == 1;
-        for (int t = blockIdx.x, k = 0; t < nt; t += gridDim.x, k++) {
-            if (k < 64 && (done >> k & 1)) continue;
-            const int still = extend_tile(g, a, w, L, w.tiles_ext[t / kExtPerTile], t % kExtPerTile,
-                                          p == 0 && round == 0, one ? kPatienceLast : kPatienceMany);
-            if (still) open++;
-            else if (k < 64) done |= 1ull << k;
-        }
-        if (!open || one) break;
+    if ((int)blockIdx.x >= nt) return;
+    const bool many = __builtin_amdgcn_readfirstlane(nt > (int)gridDim.x);
+    // the first tile is the workgroup's own, the others go by ticket
+    if (threadIdx.x == 0) {
+        L.held[0] = blockIdx.x;
+        L.patience = many ? kPatienceTake : kPatienceLast;
+        L.t = L.k = L.idle = L.open = 0;
+        L.heard = -2;  // not asked
+        L.nheld = 1;
+        L.moved = -1;
+        L.fresh = p == 0;
+        L.more = L.take = many;
     }
-    if (open && threadIdx.x == 0) atomicAdd(&w.cnt[kCntIter + slot], open);
+    int t = blockIdx.x;
+    bool fresh = p == 0;
+    int patience = many ? kPatienceTake : kPatienceLast;
+    while (true) {
+        extend_tile(g, a, w, L, w.tiles_ext[t / kExtPerTile], t % kExtPerTile, fresh, many, patience);
+        if (!many) {
+            if (L.left && threadIdx.x == 0) atomicAdd(&w.cnt[kCntIter + slot], 1);
+            break;
+        }
+        if (threadIdx.x < 64) ext_next(w, L, nt, p, slot);
+        __syncthreads();
+        t = L.t;
+        if (t < 0) break;
+        fresh = L.fresh;
+        patience = L.patience;
+    }
 }
 __global__ __launch_bounds__(kExtThreads, 5) void k_extend_tiles(Grid g, ObjArrays a, LsWork w, int p, int slot) {
     extend_tiles(g, a, w, p, slot);
@@ -1285,13 +1423,13 @@ __global__ __launch_bounds__(kTileThreads) void k_ext_open_b(Grid g, const ExtIt
     const ExtItem &x = it[blockIdx.y];
     ext_open_body(g, x.a, x.w);
 }
-// Counters of a batch of solids: clear the pass slots of every solid, or
+// Counters of a batch of solids: clear the passes' tickets and slots of every solid, or
 // gather its error flags and the first `batch` slots into out (batch + 1
 // ints per solid)
 template <class Item>
 __global__ void k_batch_zero(const Item *it, int n) {
     for (int k = blockIdx.x; k < n; k += gridDim.x)
-        for (int e = threadIdx.x; e < kIterSlots; e += blockDim.x) it[k].w.cnt[kCntIter + e] = 0;
+        for (int e = threadIdx.x; e < 2 * kIterSlots; e += blockDim.x) it[k].w.cnt[kCntTicket + e] = 0;
 }
 template <class Item>
 __global__ void k_batch_gather(const Item *it, int n, int batch, int *out) {
@@ -1375,7 +1513,7 @@ int iter_enqueue(hipStream_t s, LsWork &w, int predict, int passes, F pass, int 
     batch = predict < least ? least : predict;
     if (batch > kIterSlots) batch = kIterSlots;
     if (passes || !zeroed) {
-        k_zero_counts<<<1, 64, 0, s>>>(w.cnt + kCntIter, kIterSlots);
+        k_zero_counts<<<1, 64, 0, s>>>(w.cnt + kCntTicket, 2 * kIterSlots);
         KCHECK();
     }
     for (int b = 0; b < batch; b++)
@@ -1559,6 +1697,8 @@ int ls_alloc(const Grid &g, LsWork &w, hipStream_t s) {
     HIP_CHECK(memset_sync(w.tflag, 0, T * sizeof(int), s));
     HIP_CHECK(hipMalloc((void **)&w.tiles_fim, T * sizeof(int)));
     HIP_CHECK(hipMalloc((void **)&w.tiles_ext, T * sizeof(int)));
+    HIP_CHECK(hipMalloc((void **)&w.tprog, T * sizeof(int)));
+    HIP_CHECK(memset_sync(w.tprog, 0, T * sizeof(int), s));
     HIP_CHECK(hipMalloc((void **)&w.cnt, (kCntIter + kIterSlots) * sizeof(int)));
     HIP_CHECK(hipHostMalloc((void **)&w.hcnt, (kCntIter + kIterSlots) * sizeof(int), hipHostMallocDefault));
     HIP_CHECK(hipMalloc((void **)&w.bbox, 4 * sizeof(int)));
@@ -1569,7 +1709,7 @@ int ls_alloc(const Grid &g, LsWork &w, hipStream_t s) {
 
 void ls_free(LsWork &w) {
     void *p[] = {w.va, w.vb, w.ex, w.ey, w.iface, w.mark, w.cflag, w.tflag,
-                 w.tiles_fim, w.tiles_ext, w.cnt, w.bbox};
+                 w.tiles_fim, w.tiles_ext, w.tprog, w.cnt, w.bbox};
     for (auto q : p)
         if (q) (void)hipFree(q);
     if (w.hcnt) (void)hipHostFree(w.hcnt);
@@ -1930,16 +2070,18 @@ void ls_reset_window(LsWork &w) {
     w.have_win = false;
 }
 
-// Workgroups per solid of an extension: enough that a solid's tiles all wait
-// for each other on the GPU at once (four of these workgroups fit a CU, 1024
-// the chip). Of several solids the first ones' workgroups are dispatched
-// first, so a solid whose tiles are all resident is always among them.
-constexpr int kExtBlocks = 1024;
-static int ext_blocks(size_t n) { return std::max(128, kExtBlocks / std::max(1, (int)(n + 3) / 4)); }
+// Workgroups per solid of an extension. A lone solid gets as many as run on the
+// GPU at once (three of these workgroups fit a CU): every one holds its tiles
+// from the start, none waits for one that has not been dispatched (with 1024
+// a band 60 cells wide, 917 tiles, takes 2 to 8 ms in up to 10 launches, now 1.6).
+// Of several solids the first ones' workgroups are dispatched first, so a
+// solid whose tiles are all held is always among them.
+constexpr int kExtBlocks = 768, kExtBlocksBatch = 1024;
+static int ext_blocks_batch(size_t n) { return std::max(128, kExtBlocksBatch / std::max(1, (int)(n + 3) / 4)); }
 constexpr int kMaxExtPasses = 4096;
 
 int ls_extend(hipStream_t s, const Grid &g, const ObjArrays &a, LsWork &w, int *ext_iters) {
-    const int nb = ext_blocks(1);
+    const int nb = kExtBlocks;
     k_ext_open<<<nb, kTileThreads, 0, s>>>(g, a, w);
     KCHECK();
     int passes = 0;
@@ -1964,7 +2106,7 @@ int ls_extend_batch(hipStream_t s, const Grid &g, const std::vector<LsJob> &jobs
         items.push_back(ExtItem{*jobs[k].a, *jobs[k].w});
         pred.push_back(&jobs[k].w->pred_ext);
     }
-    const int nb = ext_blocks(n);
+    const int nb = ext_blocks_batch(n);
     std::vector<int> passes;
     const int rc = iterate_batch(s, bt, items, pred, kMaxExtPasses, [&](int p, int slot, const ExtItem *dd, int m) -> int {
         if (p == 0) {
