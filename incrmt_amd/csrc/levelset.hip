@@ -86,8 +86,6 @@ constexpr int kListBlocks = 1024;
 constexpr int kNewtonThreads = 64;  // a wavefront a workgroup: the few there are spread over the chip
 constexpr int kTileBlocks = 512;
 
-inline dim3 grid2(int nx, int ny) { return dim3((nx + BX - 1) / BX, (ny + BY - 1) / BY); }
-
 __device__ inline void ls_coords(const Grid &g, int ij, int &I, int &J) {
     const int r = ij - (kOrigin - 2);
     J = r / g.P;
@@ -663,8 +661,8 @@ __global__ __launch_bounds__(kTileThreads) void k_fim_tiles_batch(Grid g, EikGeo
 
 // Final band (levelset.cc:300-335, 408-413): accepted points get their
 // fixed-point values and status 5/2, points the heap would have left in its
-// queue status 6/1, everything outside the band the cut-off value. Outside
-// band points are listed for the extension.
+// queue status 6/1, everything outside the band the cut-off value. Tiles with
+// outside band points are flagged for the extension.
 // Bound by latency: a thread's four points share their neighbours' rows, every
 // load is issued before the first test (29.6 -> 12.7 us for a circle
 // on 1024^2), the band's box is formed from votes, and an atomic goes out only

@@ -843,8 +843,8 @@ __global__ void k_coarse_solve(int kind, LevelArgs a, FemC k, T *z, T *b, const 
 // With a division in every phase, the coefficients re-read in each, run-time
 // branches on the kind and the coarsest level eliminated in every cycle, a
 // cycle of 32^2 and 33^2 points took 33.3 us on average in double precision;
-// now 14.6 (MAC) and 23.9 us (FEM), in single precision 32.2 -> 15.9 and 25.9,
-// periodic 40.1 -> 22.1 and 33.0. A phase of one
+// now 15.0 (MAC) and 23.9 us (FEM), in single precision 32.2 -> 16.0 and 25.2,
+// periodic (a 360^2 box) 40.1 -> 21.5 and 26.6. A phase of one
 // wavefront is about 340 (MAC) to 400 cycles (FEM), a visit's start and
 // transfer about 1200.
 constexpr int kTailMaxLev = 12;
@@ -975,8 +975,8 @@ __global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs A) {
     // Offsets from a point to its periodic mirrors (put_mirrors'), 0 where it has
     // none: found once a visit, not at every write, and a mirror write is one
     // branch (a place written twice gets the same value). With the own block's
-    // registers (off_fem) a FEM cycle of a 360^2 box takes 25.8 us instead of
-    // 32.7, a MAC cycle 21.4 instead of 22.3.
+    // registers (off_fem) that took 6 us off a FEM cycle of a 360^2 box, 0.8 off a
+    // MAC cycle.
     auto mirror_x = [&](const Lv &L, int i) -> int {
         return PER && px && (i == 0 || i == L.v.nx - 1) ? (i == 0 ? L.v.nx : -L.v.nx) : 0;
     };
@@ -1937,8 +1937,9 @@ __global__ void k_copy_level(LevelArgs a, const double *z, double *zp) {
 // in e's place). Each neighbour's new value is formed again from z and e, with
 // k_add_f32's and k_residual_f32's expressions. Memory bound: 60 bytes a MAC
 // point in two passes become 52 in one, with the norms 92 in three passes 52
-// (FEM 52 and 76 become 44). At 1024^2 13.6 us MAC, 17.1 FEM, 16.4 and 20.0
-// with the norms; 24 steps of a fluid at 1024^2 70.1 -> 69.1 ms.
+// (FEM 52 and 76 become 44). At 1024^2 13.6 us MAC, 17.1 FEM, and 21.5 and 24.1
+// with the norms and their sum over the workgroups; 24 steps of a fluid at 1024^2
+// 70.1 -> 69.1 ms.
 template <int KIND>
 __device__ __forceinline__ double mixed_point(const LevelArgs &a, const FemC &k, const double *z, const float *e,
                                               const double *b, const double *c1, const double *c2, double *z2, float *bf,
