@@ -886,6 +886,7 @@ struct ExtLds {
     unsigned short halo[kEN];        // the halo points to poll
     int nhalo, left, stop;
     unsigned news;                   // counts values that have become final here
+    unsigned quit;                   // what it was when the first wavefront gave up
     int was;                         // points open before the visit
     // ext_next's state: the visit (tile number, -1: none; its place in held,
     // ext_news before it), the tiles held and ext_news before their last
@@ -943,7 +944,10 @@ __device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, c
         }
     }
     if (tid < kEHt) L.need[tid] = 0;
-    if (tid == 0) L.nhalo = L.left = L.stop = L.news = 0;
+    if (tid == 0) {
+        L.nhalo = L.left = L.stop = L.news = 0;
+        L.quit = ~0u;
+    }
 #pragma unroll
     for (int u = 0; u < kRounds; u++) {
         const int r = fr + u * kRowsAtOnce, s = rst[u];
@@ -1220,7 +1224,10 @@ __device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, c
                     __builtin_amdgcn_s_sleep(1);
                     end = lds_now(L.stop);
                 } while (!end && !far && lds_now(L.news) == news);
-                if (end) break;
+                if (end) {
+                    if (lane == 0) atomicMin(&L.quit, news);
+                    break;
+                }
                 continue;
             }
             lds_order();
@@ -1314,7 +1321,9 @@ __device__ __forceinline__ void ext_next(const LsWork &w, ExtLds &L, int nt, int
         idle += kPatienceMany;
     }
     if (left) {
-        if (first) L.seen[k] = L.heard;
+        // (a wavefront that gave up before the last values came here may have
+        // points that are ready now)
+        if (first) L.seen[k] = L.quit == L.news ? L.heard : -2;
         k++;
     } else {  // the last one takes its place
         held--;

@@ -1,10 +1,10 @@
 """The extension ends in about one launch however its tiles depend on each
 other: the tiles of a lattice of blobs and of bands many tiles deep, more of them
-than workgroups, bit for bit against the oracle's serial extrapolate_fields.
+than workgroups, also where fits' windows grow (spacings of a few 1e-6), bit for
+bit against the oracle's serial extrapolate_fields.
 Every tile is held by a workgroup that runs, so one launch is enough; the
 bound leaves room for a workgroup that gave up early. (Sweeps over all tiles
-take a launch for each tile boundary on the longest chain: 20, 113 and about 150
-here.)"""
+take a launch for each tile boundary on the longest chain: 16 to about 150 here.)"""
 import numpy as np
 import pytest
 
@@ -26,10 +26,10 @@ def _blobs(x, y):
     return 50 / np.pi * (0.35 + 0.03 * np.sin(0.013 * x + 0.02 * y) - np.cos(np.pi * x / 50) * np.cos(np.pi * y / 50))
 
 
-@pytest.mark.parametrize("m,n,shape,cells,tiles", [
-    (63, 50, wavy, 7.0, 1), (803, 811, _blobs, 6.0, 1500), (700, 700, _star(200, 30), 100.0, 769),
-    (1200, 1180, _star(340, 50), 160.0, 1900)])
-def test_about_one_launch(m, n, shape, cells, tiles):
-    s, passes = _compare(m, n, 2.0 / 800, shape, cells)
+@pytest.mark.parametrize("m,n,h,shape,cells,tiles", [
+    (63, 50, 2.5e-3, wavy, 7.0, 1), (803, 811, 2.5e-3, _blobs, 6.0, 1500), (700, 700, 2.5e-3, _star(200, 30), 100.0, 769),
+    (1200, 1180, 2.5e-3, _star(340, 50), 160.0, 1900), (803, 811, 8e-6, _blobs, 5.0, 1500)])
+def test_about_one_launch(m, n, h, shape, cells, tiles):
+    s, passes = _compare(m, n, h, shape, cells)
     assert _tiles(s, m, n) >= tiles
     assert passes <= 4
