@@ -893,6 +893,7 @@ struct ExtLds {
     // visits (-1: none yet)
     int t, k, heard, patience, nheld, open, idle, moved;
     bool fresh, more, take;
+    bool wide;                       // a point's fit is of a larger radius
     int held[kExtHeld], seen[kExtHeld];
 };
 
@@ -947,6 +948,7 @@ __device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, c
     if (tid == 0) {
         L.nhalo = L.left = L.stop = L.news = 0;
         L.quit = ~0u;
+        L.wide = false;
     }
 #pragma unroll
     for (int u = 0; u < kRounds; u++) {
@@ -991,16 +993,12 @@ __device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, c
         jlo = j <= r ? -j : -r; jhi = j + r >= nn ? nn - 1 - j : r;
     };
     // A fit of a larger radius (none in the usual shapes: the moments of a
-    // radius-3 window are far from singular) reaches past the halo and reads
-    // the grid itself: whether it reads point p, and the weight.
-    auto reads = [&](int p, double &wgt) {
-        const int s = a.st[p];
-        if (s < 2 || s > 5) return false;
-        wgt = a.phi[p];
-        if (!(wgt < pp)) return false;
-        wgt = pp - wgt;
-        return true;
-    };
+    // radius-3 window are far from singular unless the spacing is below about
+    // 1e-5) reaches past the halo and reads the grid itself. Its mask holds one of
+    // the outside points that it reads: the last in phi, mostly the last to be
+    // final, and so the one to wait for (looking at the whole window, up to 225
+    // points, at every poll instead took 3.1 ms for 13 tiles at 61 x 66 and spacing
+    // 8e-6, now 0.32, and 49 ms for a band 40 cells deep on 700 x 690, now 1.9).
     if (todo) {
         // the radius-3 window, unrolled a row at a time; window points
         // outside the grid hold status -1, which the status test rejects, so
@@ -1038,13 +1036,24 @@ __device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, c
                 int ilo, ihi, jlo, jhi;
                 window(rr, ilo, ihi, jlo, jhi);
                 S = Sx = Sy = Sxx = Sxy = Syy = 0;
-                for (int dj = jlo; dj <= jhi; dj++)
+                int last = -1;
+                double least = INFINITY;
+                for (int dj = jlo; dj <= jhi; dj++) {
+                    const int p0 = q + dj * g.P;
+#pragma unroll 1  // unrolled, it costs the loop below its registers
                     for (int di = ilo; di <= ihi; di++) {
-                        double wgt;
-                        if (!reads(q + dj * g.P + di, wgt)) continue;
+                        const int s = a.st[p0 + di];  // read with phi, whatever it is
+                        const double ph = a.phi[p0 + di], wgt = pp - ph;
+                        if (s < 2 || s > 5 || !(ph < pp)) continue;
                         S += wgt; Sx += di * wgt; Sy += dj * wgt;
                         Sxx += di * di * wgt; Sxy += di * dj * wgt; Syy += dj * dj * wgt;
+                        if (s >= 4 && wgt < least) {
+                            least = wgt;
+                            last = p0 + di;
+                        }
                     }
+                }
+                mask = (unsigned)last;
                 det = S * (Sxy * Sxy - Sxx * Syy) + Sx * Sx * Syy - 2 * Sx * Sxy * Sy + Sy * Sy * Sxx;
                 rr++;
             } while (fabs(det) < 1e-10 && rr <= 7);
@@ -1069,6 +1078,7 @@ __device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, c
             }
         }
     }
+    if (todo && wide) L.wide = true;
     const unsigned long long open = __ballot(todo);
     if (lane == 0 && open) atomicAdd(&L.left, __popcll(open));
     __syncthreads();
@@ -1096,6 +1106,8 @@ __device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, c
             hp[u] = k < nh ? L.halo[k] : -1;
             at[u] = hp[u] < 0 ? 0 : g.ls(I0 + hp[u] % kEW, J0 + hp[u] / kEW);
         }
+        // (a visit of larger windows takes long to set up)
+        const int enough = L.wide && patience < kPatienceTake ? kPatienceTake : patience;
         int seen = -1, idle = 0, moved = -1;
         while (true) {
             unsigned long long px[kOwn], py[kOwn];
@@ -1124,7 +1136,7 @@ __device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, c
                 if (((lf ^ seen) & -kTellPoints) && lane == 0) ext_tell(w);
                 seen = lf;
                 idle = 0;
-            } else if (++idle > patience) {
+            } else if (++idle > enough) {
                 const int now = patience == kPatienceLast ? ext_moved(w) : moved;
                 if (now == moved) {
                     if (lane == 0) atomicOr(&L.stop, 1);
@@ -1191,86 +1203,113 @@ __device__ __forceinline__ void extend_tile(const Grid &g, const ObjArrays &a, c
             // path shares, would also wait for that path's last stores
             __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
         };
-        while (__any(todo)) {
-            const unsigned news = lds_now(L.news);
-            lds_order();
-            bool ready = false;
-            if (todo && !wide) {
-                // (plain reads, issued together: one after the other they
-                // took half of a link's time)
-                unsigned k[7], miss = 0;
+        // the points of this wavefront; by itself where none has a larger window,
+        // whose code would cost that loop registers
+        auto work = [&](auto larger) {
+            constexpr bool WIDE = decltype(larger)::value;
+            while (__any(todo)) {
+                const unsigned news = lds_now(L.news);
+                lds_order();
+                bool ready = false;
+                if (todo && !(WIDE && wide)) {
+                    // (plain reads, issued together: one after the other they
+                    // took half of a link's time)
+                    unsigned k[7], miss = 0;
 #pragma unroll
-                for (int b = 0; b < 7; b++) k[b] = L.known[lj + b - 3];
+                    for (int b = 0; b < 7; b++) k[b] = L.known[lj + b - 3];
 #pragma unroll
-                for (int b = 0; b < 7; b++) miss |= (unsigned)(mask >> (7 * b)) & 127u & ~(k[b] >> (li - 3));
-                ready = !miss;
-            }
-            const unsigned long long far = __ballot(todo && wide);
-            for (unsigned long long b = far; b; b &= b - 1) {
-                const int l = __ffsll((long long)b) - 1;
-                bool miss = false;
-                each_wide(l, 64, [&](bool in, int p, int st, double, int, int) {
-                    if (in && st >= 4) miss |= ext_load(w.ex + p) == kExtOpen || ext_load(w.ey + p) == kExtOpen;
-                });
-                if (!__any(miss) && lane == l) ready = true;
-            }
-            const unsigned long long rd = __ballot(ready);
-            if (!rd) {
-                // nothing to do until another value is final: a spin on one
-                // word leaves the SIMD to the wavefronts that work (a larger
-                // window waits for values outside the tile too)
-                int end = 0;
-                do {
-                    __builtin_amdgcn_s_sleep(1);
-                    end = lds_now(L.stop);
-                } while (!end && !far && lds_now(L.news) == news);
-                if (end) {
-                    if (lane == 0) atomicMin(&L.quit, news);
-                    break;
+                    for (int b = 0; b < 7; b++) miss |= (unsigned)(mask >> (7 * b)) & 127u & ~(k[b] >> (li - 3));
+                    ready = !miss;
                 }
-                continue;
-            }
-            lds_order();
-            for (unsigned long long b = rd; b; b &= b - 1) {
-                const int l = __ffsll((long long)b) - 1;
-                double sum = 0;
-                if (!(far >> l & 1)) {
-                    const int el = __builtin_amdgcn_readlane(e, l);
-                    const unsigned mlo = __builtin_amdgcn_readlane((unsigned)mask, l),
-                                   mhi = __builtin_amdgcn_readlane((unsigned)(mask >> 32), l);
-                    add_up(lane < 49 && ((lane < 32 ? mlo >> lane : mhi >> (lane - 32)) & 1), L.phi[el] - L.phi[el + off],
-                           xx, yy, L.x[el + off], L.y[el + off], sum);
-                } else {
-                    each_wide(l, 48, [&](bool in, int p, int st, double wgt, int cx, int cy) {
-                        double fa = 0, fb = 0;
-                        if (in) {
-                            fa = st >= 4 ? __longlong_as_double((long long)ext_load(w.ex + p)) : a.nX[p];
-                            fb = st >= 4 ? __longlong_as_double((long long)ext_load(w.ey + p)) : a.nY[p];
-                        }
-                        add_up(in, wgt, cx, cy, fa, fb, sum);
-                    });
+                const unsigned long long far = WIDE ? __ballot(todo && wide) : 0;
+                if (WIDE && todo && wide) {
+                    const int p = (int)(unsigned)mask;
+                    ready = p < 0 || (ext_load(w.ex + p) != kExtOpen && ext_load(w.ey + p) != kExtOpen);
                 }
-                const double p0 = lane_double(sum, 0), p1 = lane_double(sum, 1), p2 = lane_double(sum, 2),
-                             p3 = lane_double(sum, 3), p4 = lane_double(sum, 4), p5 = lane_double(sum, 5);
-                if (lane == l) {
-                    const double vx = p0 * al + p1 * be + p2 * ga, vy = p3 * al + p4 * be + p5 * ga;
-                    L.x[e] = vx;
-                    L.y[e] = vy;
-                    lds_order();
-                    atomicOr(&L.known[lj], 1u << li);
-                    atomicAdd(&L.news, 1u);
-                    ext_store(w.ex + q, vx);
-                    ext_store(w.ey + q, vy);
-                    if (store) {
-                        a.nX[q] = vx;
-                        a.nY[q] = vy;
+                const unsigned long long rd = __ballot(ready);
+                if (!rd) {
+                    // nothing to do until another value is final: a spin on one
+                    // word leaves the SIMD to the wavefronts that work (a larger
+                    // window waits for values outside the tile too)
+                    int end = 0;
+                    do {
+                        __builtin_amdgcn_s_sleep(1);
+                        end = lds_now(L.stop);
+                    } while (!end && !far && lds_now(L.news) == news);
+                    if (end) {
+                        if (lane == 0) atomicMin(&L.quit, news);
+                        break;
                     }
-                    todo = false;
+                    continue;
                 }
+                lds_order();
+                unsigned long long done = rd;
+                for (unsigned long long b = rd; b; b &= b - 1) {
+                    const int l = __ffsll((long long)b) - 1;
+                    double sum = 0;
+                    if (!WIDE || !(far >> l & 1)) {
+                        const int el = __builtin_amdgcn_readlane(e, l);
+                        const unsigned mlo = __builtin_amdgcn_readlane((unsigned)mask, l),
+                                       mhi = __builtin_amdgcn_readlane((unsigned)(mask >> 32), l);
+                        add_up(lane < 49 && ((lane < 32 ? mlo >> lane : mhi >> (lane - 32)) & 1), L.phi[el] - L.phi[el + off],
+                               xx, yy, L.x[el + off], L.y[el + off], sum);
+                    } else {
+                        int last = -1;  // a point that is open still: the next to wait for
+                        double least = INFINITY;
+                        each_wide(l, 48, [&](bool in, int p, int st, double wgt, int cx, int cy) {
+                            double fa = 0, fb = 0;
+                            if (in && st >= 4) {
+                                const unsigned long long bx = ext_load(w.ex + p), by = ext_load(w.ey + p);
+                                fa = __longlong_as_double((long long)bx);
+                                fb = __longlong_as_double((long long)by);
+                                if ((bx == kExtOpen || by == kExtOpen) && wgt < least) {
+                                    least = wgt;
+                                    last = p;
+                                }
+                            } else if (in) {
+                                fa = a.nX[p];
+                                fb = a.nY[p];
+                            }
+                            add_up(in, wgt, cx, cy, fa, fb, sum);
+                        });
+                        if (__any(last >= 0)) {
+                            for (int h = 32; h > 0; h /= 2) {
+                                const double o = __shfl_xor(least, h, 64);
+                                const int po = __shfl_xor(last, h, 64);
+                                if (o < least) {
+                                    least = o;
+                                    last = po;
+                                }
+                            }
+                            if (lane == l) mask = (unsigned)last;
+                            done &= ~(1ull << l);
+                            continue;
+                        }
+                    }
+                    const double p0 = lane_double(sum, 0), p1 = lane_double(sum, 1), p2 = lane_double(sum, 2),
+                                 p3 = lane_double(sum, 3), p4 = lane_double(sum, 4), p5 = lane_double(sum, 5);
+                    if (lane == l) {
+                        const double vx = p0 * al + p1 * be + p2 * ga, vy = p3 * al + p4 * be + p5 * ga;
+                        L.x[e] = vx;
+                        L.y[e] = vy;
+                        lds_order();
+                        atomicOr(&L.known[lj], 1u << li);
+                        atomicAdd(&L.news, 1u);
+                        ext_store(w.ex + q, vx);
+                        ext_store(w.ey + q, vy);
+                        if (store) {
+                            a.nX[q] = vx;
+                            a.nY[q] = vy;
+                        }
+                        todo = false;
+                    }
+                }
+                if (lane == 0) atomicSub(&L.left, __popcll(done));
+                if (many && lane == 0 && done) (void)__hip_atomic_fetch_add(&w.tprog[tile], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            if (lane == 0) atomicSub(&L.left, __popcll(rd));
-            if (many && lane == 0) (void)__hip_atomic_fetch_add(&w.tprog[tile], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        };
+        if (__any(todo && wide)) work(std::true_type());
+        else work(std::false_type());
     }
     __syncthreads();
 }

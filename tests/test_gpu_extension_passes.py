@@ -28,7 +28,9 @@ def _blobs(x, y):
 
 @pytest.mark.parametrize("m,n,h,shape,cells,tiles", [
     (63, 50, 2.5e-3, wavy, 7.0, 1), (803, 811, 2.5e-3, _blobs, 6.0, 1500), (700, 700, 2.5e-3, _star(200, 30), 100.0, 769),
-    (1200, 1180, 2.5e-3, _star(340, 50), 160.0, 1900), (803, 811, 8e-6, _blobs, 5.0, 1500)])
+    (1200, 1180, 2.5e-3, _star(340, 50), 160.0, 1900), (250, 260, 8e-6, _star(70, 12), 7.0, 40),
+    (700, 690, 4e-6, _star(200, 30), 40.0, 300), (803, 811, 8e-6, _blobs, 5.0, 1500),
+    (1400, 1400, 8e-6, _star(400, 60), 60.0, 769)])
 def test_about_one_launch(m, n, h, shape, cells, tiles):
     s, passes = _compare(m, n, h, shape, cells)
     assert _tiles(s, m, n) >= tiles
