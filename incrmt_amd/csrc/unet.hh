@@ -56,6 +56,16 @@ struct ConvSpec {
     size_t w_off, b_off;  // offsets into the master parameter array (floats)
 };
 
+// A layer's weight and bias gradient as its workgroups' sums.
+struct DwSum {
+    const float *part = nullptr;
+    int tiles = 0, nci = 0, nco = 0, chunks = 0;  // chunks 0: nothing to add up
+    int cin = 0, cout = 0, kp = 0;
+    float *dw = nullptr, *db = nullptr;           // [cout_p][kp], [cout]
+    // workgroups that adding them up takes
+    __host__ __device__ int blocks() const { return chunks ? tiles * 9 * 16 + nco : 0; }
+};
+
 class UNet {
   public:
     ~UNet();
@@ -111,6 +121,8 @@ class UNet {
     float *gact_[kUnetLayers] = {nullptr};    // d loss / d layer output
     float *gup_[3] = {nullptr};
     bf16_t *dpre_ = nullptr;                  // masked output gradient of the layer in hand (bf16)
+    float *dw_part_ = nullptr;                // the weight-gradient sums of its workgroups
+    DwSum dw_sum_;                            // what is left to add up of them
     const bf16_t *last_in_ = nullptr;         // input of the last forward pass
     double *d_loss_ = nullptr;
     double *h_loss_ = nullptr;

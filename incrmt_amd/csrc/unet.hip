@@ -212,8 +212,8 @@ struct DwArgs {
     int nco, nci;         // 16-blocks of output and input channels
     long long segs;       // 16-node row segments of the output grid
     int seg_chunk;        // segments per workgroup
-    float *dw;            // [cout_p][kp]
-    float *db;            // [cout]: the bias gradient (workgroups of input block 0 add it)
+    float *part;          // the workgroups' tiles: [seg chunk][block pair][tap][256], then
+                          // the bias sums of input block 0: [seg chunk][output block][16]
 };
 
 // dW of one (output-channel block, input-channel block) pair for all nine
@@ -222,8 +222,9 @@ struct DwArgs {
 // 8-byte channel-quad loads, transposes them through its own LDS slots
 // (the MFMA wants four consecutive nodes of one channel per lane), and
 // accumulates one MFMA per tap. The four wavefronts' tiles are summed in
-// LDS and added to dW. The workgroups of input block 0 also sum dpre over
-// their nodes for the bias gradient.
+// LDS and written out; sum_dw adds up the workgroups' in their order. The
+// workgroups of input block 0 also sum dpre over their nodes for the bias
+// gradient.
 __global__ __launch_bounds__(kThreads) void k_conv_dw(DwArgs a) {
     __shared__ bf16_t ta[4][256], tb[4][256];
     __shared__ float red[4][256];
@@ -276,14 +277,13 @@ __global__ __launch_bounds__(kThreads) void k_conv_dw(DwArgs a) {
         __builtin_amdgcn_wave_barrier();
     }
     // D row = output channel 4 kg + i of the block, column = input channel pl
-    const int e = threadIdx.x, r = e >> 4, cc = e & 15;
-    const int gco = cob * 16 + r, gci = cib * 16 + cc;
+    const int e = threadIdx.x;
+    const size_t wg = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
     for (int t = 0; t < 9; t++) {
 #pragma unroll
         for (int i = 0; i < 4; i++) red[wave][(4 * kg + i) * 16 + pl] = acc[t][i];
         __syncthreads();
-        const float v = red[0][e] + red[1][e] + red[2][e] + red[3][e];
-        if (gco < a.cout && gci < cin && v != 0.f) atomicAdd(&a.dw[(size_t)gco * a.kp + kidx(t, gci)], v);
+        a.part[(wg * 9 + t) * 256 + e] = red[0][e] + red[1][e] + red[2][e] + red[3][e];
         __syncthreads();
     }
     if (cib != 0) return;
@@ -295,17 +295,54 @@ __global__ __launch_bounds__(kThreads) void k_conv_dw(DwArgs a) {
         float b = 0.f;
         for (int w = 0; w < 4; w++)
             for (int n = 0; n < 16; n++) b += red[w][threadIdx.x * 16 + n];
-        const int ch = cob * 16 + threadIdx.x;
-        if (ch < a.cout && b != 0.f) atomicAdd(&a.db[ch], b);
+        a.part[(size_t)gridDim.y * gridDim.x * 2304 + ((size_t)blockIdx.y * a.nco + cob) * 16 + threadIdx.x] = b;
     }
 }
 
+// The weight and bias gradients of a layer from its workgroups' sums, added in
+// a fixed order (atomics gave other bits on every call, and a network trained on
+// them other weights). Workgroup b takes 16 of a tile's 256 entries (or 16
+// biases): 16 threads an entry, each every 16th segment chunk, then those in
+// order. The sums of one layer ride on the next layer's k_relu_bwd launch. A pass at
+// 257^2 takes 182 us in k_conv_dw, 62 in k_relu_bwd and 5 in k_sum_dw, with atomics and
+// a fill before them 203, 56 and 2.
+__device__ void sum_dw(const DwSum &a, int b) {
+    __shared__ float s[16][17];
+    const int c = threadIdx.x & 15, g = threadIdx.x >> 4;
+    const bool bias = b >= a.tiles * 9 * 16;
+    const int ub = bias ? b - a.tiles * 9 * 16 : b;
+    const size_t step = bias ? (size_t)a.nco * 16 : (size_t)a.tiles * 2304;
+    const float *p = a.part + (bias ? (size_t)a.chunks * a.tiles * 2304 + ub * 16 : (size_t)ub * 16) + c;
+    float v = 0.f;
+#pragma unroll 8
+    for (int k = g; k < a.chunks; k += 16) v += p[k * step];
+    s[g][c] = v;
+    __syncthreads();
+    if (g != 0) return;
+    v = 0.f;
+    for (int k = 0; k < 16; k++) v += s[k][c];
+    if (bias) {
+        if (ub * 16 + c < a.cout) a.db[ub * 16 + c] = v;
+        return;
+    }
+    const int tile = ub / 144, t = ub / 16 % 9, e = ub % 16 * 16 + c;
+    const int gco = tile / a.nci * 16 + (e >> 4), gci = tile % a.nci * 16 + (e & 15);
+    if (gco < a.cout && gci < a.cin) a.dw[(size_t)gco * a.kp + kidx(t, gci)] = v;
+}
+
+__global__ __launch_bounds__(kThreads) void k_sum_dw(DwSum a) { sum_dw(a, blockIdx.x); }
+
 // dpre = d loss / d (pre-activation) in BF16: the output gradient where the
-// ReLU passed (act > 0), zero elsewhere and on the padding channels
-__global__ void k_relu_bwd(const bf16_t *act, const float *g, int cout, int cd, long long npix, int relu,
-                           bf16_t *dpre) {
+// ReLU passed (act > 0), zero elsewhere and on the padding channels, by the
+// first nb workgroups; the others sum the layer before's weight gradient
+__global__ __launch_bounds__(kThreads) void k_relu_bwd(const bf16_t *act, const float *g, int cout, int cd,
+                                                       long long npix, int relu, bf16_t *dpre, int nb, DwSum before) {
+    if ((int)blockIdx.x >= nb) {
+        sum_dw(before, blockIdx.x - nb);
+        return;
+    }
     const long long n = npix * cd;
-    for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < n; q += (long long)gridDim.x * blockDim.x) {
+    for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < n; q += (long long)nb * blockDim.x) {
         const long long p = q / cd;
         const int c = (int)(q - p * cd);
         float v = 0.f;
@@ -443,10 +480,6 @@ __global__ void k_build_wt(const float *w, int kp, int cin, int cout, int rows, 
         wt[q] = f2bf(v);
     }
 }
-__global__ void k_fill_f32(float *p, long long n, float v) {
-    for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < n; q += (long long)gridDim.x * blockDim.x)
-        p[q] = v;
-}
 __global__ void k_pack_input(const float *in3, long long npix, bf16_t *in4) {
     for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < npix * 4;
          q += (long long)gridDim.x * blockDim.x) {
@@ -484,6 +517,13 @@ int UNet::alloc(void **p, size_t bytes) {
     HIP_CHECK(memset_sync(*p, 0, bytes, s_));
     allocs_.push_back(*p);
     return 0;
+}
+
+// Segments of a weight-gradient workgroup: about 1024 workgroups in all, each
+// over at least 16 segments.
+static int dw_chunk(long long segs, int tiles) {
+    const long long want = (1024 + tiles - 1) / tiles, chunk = (segs + want - 1) / want;
+    return (int)(chunk < 16 ? 16 : chunk);
 }
 
 int UNet::init(int nx, int ny, unsigned seed, hipStream_t s) {
@@ -538,6 +578,13 @@ int UNet::init(int nx, int ny, unsigned seed, hipStream_t s) {
     }
     gout_ = gact_[kOut];
     if (int rc = alloc((void **)&dpre_, dpre * 2)) return rc;
+    size_t part = 0;  // the largest layer's; 10 MB at the most
+    for (const ConvSpec &c : L_) {
+        const int nco = c.cout_p / 16, tiles = nco * c.groups;
+        const long long segs = (long long)((nx_[c.lout] + 15) / 16) * ny_[c.lout], per = dw_chunk(segs, tiles);
+        part = std::max(part, (size_t)((segs + per - 1) / per) * ((size_t)tiles * 2304 + nco * 16));
+    }
+    if (int rc = alloc((void **)&dw_part_, part * 4)) return rc;
     for (int u = 0; u < 3; u++) {  // inputs of kU2 (level 2), kU1 (1), kU0 (0)
         const int lev = 2 - u, C = kUnetCh[lev + 1];
         if (int rc = alloc((void **)&up_[u], npix(lev) * C * 2)) return rc;
@@ -619,7 +666,7 @@ int UNet::conv_forward(int l, const bf16_t *in1, const bf16_t *in2, bf16_t *out_
 }
 
 // Backward through layer l: dpre from the output gradient (and the ReLU
-// mask), then dW and db (accumulated into g32_), then, when gin1 is given,
+// mask), then dW and db (as sums of workgroups, dw_sum_), then, when gin1 is given,
 // the input gradients (gin1 for the first input, gin2 for the skip input of
 // a decoder layer), added to what the buffers hold when accum is set.
 int UNet::conv_backward(int l, const bf16_t *in1, const bf16_t *in2, const bf16_t *act_out, const float *gout,
@@ -627,24 +674,25 @@ int UNet::conv_backward(int l, const bf16_t *in1, const bf16_t *in2, const bf16_
     const ConvSpec &c = L_[l];
     const long long npo = (long long)nx_[c.lout] * ny_[c.lout];
     const int cd = cd_of(c.cout);
-    k_relu_bwd<<<blocks_for(npo * cd), kThreads, 0, s_>>>(act_out, gout, c.cout, cd, npo, c.relu ? 1 : 0, dpre_);
+    const int nb = blocks_for(npo * cd);
+    k_relu_bwd<<<nb + dw_sum_.blocks(), kThreads, 0, s_>>>(act_out, gout, c.cout, cd, npo, c.relu ? 1 : 0, dpre_, nb,
+                                                          dw_sum_);
     UCHECK();
     // weights
     DwArgs d{};
     d.dpre = dpre_; d.cd = cd; d.in1 = in1; d.in2 = in2; d.c1 = c.cin1; d.c2 = c.cin2;
     d.inx = nx_[c.lin]; d.iny = ny_[c.lin]; d.onx = nx_[c.lout]; d.ony = ny_[c.lout]; d.stride = c.stride;
-    d.kp = c.kp; d.cout = c.cout; d.db = g32_ + c.b_off;
+    d.kp = c.kp; d.cout = c.cout;
     d.nco = c.cout_p / 16; d.nci = (c.cin1 + c.cin2 + 15) / 16;
     d.segs = (long long)((d.onx + 15) / 16) * d.ony;
-    // about 1024 workgroups in all, each over at least 16 segments
     const int tiles = d.nco * d.nci;
-    long long want = (1024 + tiles - 1) / tiles;
-    long long chunk = (d.segs + want - 1) / want;
-    d.seg_chunk = (int)(chunk < 16 ? 16 : chunk);
-    d.dw = g32_ + c.w_off;
-    const long long chunks = (d.segs + d.seg_chunk - 1) / d.seg_chunk;
-    k_conv_dw<<<dim3(tiles, (unsigned)chunks), kThreads, 0, s_>>>(d);
+    d.seg_chunk = dw_chunk(d.segs, tiles);
+    const int chunks = (int)((d.segs + d.seg_chunk - 1) / d.seg_chunk);
+    d.part = dw_part_;
+    k_conv_dw<<<dim3(tiles, chunks), kThreads, 0, s_>>>(d);
     UCHECK();
+    dw_sum_ = DwSum{dw_part_, tiles, d.nci, d.nco, chunks, c.cin1 + c.cin2, c.cout, c.kp, g32_ + c.w_off,
+                    g32_ + c.b_off};
     if (!gin1) return 0;
     // input gradients: the transposed convolution
     const int cin = c.cin1 + c.cin2;
@@ -707,9 +755,9 @@ int UNet::backward(const float *d_target, double *loss) {
 
 int UNet::backward_grad(const float *gout) {
     if (!last_in_) return INCRMT_ERR_ARG;
-    k_fill_f32<<<blocks_for(nmaster_), kThreads, 0, s_>>>(g32_, (long long)nmaster_, 0.f);
-    UCHECK();
+    // every parameter's gradient is written (the padding's stay zero)
     int rc;
+    dw_sum_ = DwSum{};
     // decoder: Out, then U0 (up0 | e0), U1, U2, each followed by the adjoint
     // of the up-sampling that fed it
     if ((rc = conv_backward(kOut, act_[kU0], nullptr, nullptr, gout, gact_[kU0], nullptr, false))) return rc;
@@ -734,7 +782,10 @@ int UNet::backward_grad(const float *gout) {
     for (const Step &st : steps)
         if ((rc = conv_backward(st.l, act_[st.in], nullptr, act_[st.l], gact_[st.l], gact_[st.in], nullptr, st.accum)))
             return rc;
-    return conv_backward(kE0a, last_in_, nullptr, act_[kE0a], gact_[kE0a], nullptr, nullptr, false);
+    if ((rc = conv_backward(kE0a, last_in_, nullptr, act_[kE0a], gact_[kE0a], nullptr, nullptr, false))) return rc;
+    k_sum_dw<<<dw_sum_.blocks(), kThreads, 0, s_>>>(dw_sum_);
+    UCHECK();
+    return 0;
 }
 
 int UNet::adam(float lr) {
